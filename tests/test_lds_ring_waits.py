@@ -155,6 +155,35 @@ def prefill_gemm_case(symbol):
         check(runs, f"prefill_gemm<{GEMM_EPI[epi]}, {wr}, {tm}, {d}> K {K} N {N}{' scaled' if scaled else ''}")
 
 
+# ---- the prefill's ring GEMM for middling runs ----
+
+
+def test_prefill_ring_reads_no_stage_before_it_lands():
+    kernels = assembly("prefill_short.hip")
+    symbols = instances(kernels, "prefill_ring")
+    assert len(symbols) >= 7, symbols  # q/k/v at both head widths, o and down at both strip heights, gate/up
+    L = layout("prefill_short.hip")
+    for symbol in symbols:
+        epi, wr, sw, tt, gk, r, d = template_args(symbol)
+        hidden, inner, heads, kv, M, M_pad = (1024, 4096, 16, 2, 300, 512) if d == 64 else (2048, 6144, 16, 2, 300, 512)
+        N = {0: (heads + 2 * kv) * d, 1: hidden, 2: 2 * inner, 3: hidden}[epi]
+        # K 1024 and 2048: a steady state of one and more turns of every ring depth.
+        for K in (1024, 2048):
+            for on in (False, True):  # the row scales (q/k/v, gate/up), the next norm's input (o, down)
+                g = dict(w=W, x=X, K=K, N=N, residual=0, out=0, mlp=0, q=0, kv=0, row_sq=0, next_gain=0, out_n=0, out_sq=0, rows=0)
+                if epi == 0:
+                    g.update(q=Q, kv=KV, row_sq=AUX if on else 0)
+                elif epi == 2:
+                    g.update(mlp=OUT, row_sq=AUX if on else 0)
+                else:
+                    g.update(residual=AUX, out=OUT, next_gain=AUX + 0x100000 if on else 0, out_n=OUT + 0x1000000, out_sq=OUT + 0x2000000)
+                a = prefill_args(L, M, M_pad, hidden, inner, heads, kv, d, 512, 8, 8)
+                NB, MB = N // 128, -(-M // (16 * tt))
+                runs = replay(kernels[symbol], [a, lr.pack(L, "GemmArgs", g), struct.pack("<i", NB), struct.pack("<i", MB)],
+                              (NB * MB, 1, 1), 256, rows_memory(M, M_pad, 8), [(0, 0, 0), (NB * MB - 1, 0, 0)])
+                check(runs, f"prefill_ring<{GEMM_EPI[epi]}, {wr}, {sw}, {tt}, {gk}, {r}, {d}> K {K}{' on' if on else ''}")
+
+
 # ---- the prefill attention ----
 
 

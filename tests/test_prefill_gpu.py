@@ -171,3 +171,30 @@ def test_nan_left_in_a_reused_block_past_the_run_never_reaches_its_outputs(ctx):
         assert np.all(np.isfinite(a)) and np.array_equal(a.view(np.uint32), b.view(np.uint32)), t
     dec.close()
     fresh.close()
+
+
+@pytest.mark.parametrize("rows,wide", [(1, False), (32, False), (8, True)])
+def test_a_run_of_any_length_alone_gives_its_bits_among_thousands(ctx, rows, wide):
+    """A short run's projections take kernels of their own (prefill_short.hip: strips by tiles a
+    wave, rings of 1, 2, 4 and 8 tiles); among thousands of positions the same rows go
+    through larger tiles. Lengths on both sides of every line between those kernels, at the decode
+    strip heights 4 and 16 (1 and 32 rows) and at VoxCPM2's widths: outputs and cache exactly
+    alike."""
+    from tgx.synth import StackSpec
+
+    lengths = (1, 16, 17, 33, 57, 128, 129, 256, 257, 300) if wide else (1, 16, 17, 32, 33, 57, 129, 193, 256, 257, 512, 513, 1025, 2049)
+    among = list(lengths) + ([2000, 2000, 2000] if wide else [2304, 2304])
+    widths = dict(hidden=2048, inner=6144, head_dim=128) if wide else {}
+    spec = StackSpec(layers=2, dtype="bf16", **widths)
+    cap = 2304
+    dec = make_decoder(ctx, spec, cap, rows=rows, slots=max(rows, len(among)))
+    x = inputs(spec, sum(among))
+    at = np.cumsum([0, *among])
+    whole = dec.prefill_runs([(r, 0, n) for r, n in enumerate(among)], x)
+    caches = [dec.read_cache(r, n) for r, n in enumerate(lengths)]
+    for r, n in enumerate(lengths):
+        print(f"[prefill] {n} positions alone, {rows} rows, wide {wide}", flush=True)
+        alone = dec.prefill(0, x[at[r] : at[r] + n], slot=r)
+        np.testing.assert_array_equal(alone, whole[at[r] : at[r] + n])
+        for got, want in zip(dec.read_cache(r, n), caches[r]):
+            np.testing.assert_array_equal(got, want)

@@ -175,6 +175,19 @@ __device__ __forceinline__ uint4 pair_blocks(const uint32_t (&a)[2], const uint3
     return make_uint4(r0[0], r1[0], r0[1], r1[1]);
 }
 
+// The sums over a column's four lanes (l, l ^ 16, l ^ 32, l ^ 48) of four values at once, each
+// (l0 + l1) + (l2 + l3): the lanes of row q of 16 get the q-th value's (v_permlane16_swap and
+// v_permlane32_swap trade the rows, three trades and adds where four sums alone take eight). The
+// same bits as v += lane_xor16(v); v += lane_xor32(v) (an addition's operands commute).
+__device__ __forceinline__ float column_sums4(float a, float b, float c, float d) {
+    const auto ab = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    const auto cd = __builtin_amdgcn_permlane16_swap(__float_as_uint(c), __float_as_uint(d), false, false);
+    const float x = __uint_as_float(ab[0]) + __uint_as_float(ab[1]);
+    const float y = __uint_as_float(cd[0]) + __uint_as_float(cd[1]);
+    const auto xy = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return __uint_as_float(xy[0]) + __uint_as_float(xy[1]);
+}
+
 // Attention's online softmax over a turn of 16 PT keys (PT 4: a 64-key block at head_dim 64; PT 2:
 // half a block at head_dim 128) for the 16 columns (query heads or (position, head) pairs) of a
 // wave, from S^T = K Q^T in s[pt] (key 16 pt + 4 (lane / 16) + i, column lane % 16) and the turn's

@@ -103,7 +103,7 @@ struct RowScale {
             total += p[i].z;
             total += p[i].w;
         }
-        return 1.0f / sqrtf(total / (float)g.K + a.eps);
+        return rms_scale(total, g.K, a.eps);
     }
 };
 
@@ -327,8 +327,8 @@ prefill_gemm(PrefillArgs a, GemmArgs g) {
     if (residual_epilogue(EPI)) {
         // The residual plus the products (EPI_RESIDUAL_IN: the accumulators hold both). With
         // next_gain: each lane's squares of its row's 32 values of the wave's 128 columns, in
-        // strip order, then the 4 lanes of a row added (lanes l ^ 16, l ^ 32). EPI_RESIDUAL loads
-        // the residual rows of four strips at once (rows past M read row M - 1, never stored).
+        // strip order, then the 4 lanes of a row added. EPI_RESIDUAL loads the residual rows of four
+        // strips at once (rows past M read row M - 1, never stored).
         float sq[WT] = {};
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
@@ -367,12 +367,7 @@ prefill_gemm(PrefillArgs a, GemmArgs g) {
                         *reinterpret_cast<float4*>(g.out + (size_t)m * g.N + n) = o;
                         normed[h][0] = pack_bf16x2(o.x * gn[s4].x, o.y * gn[s4].y);
                         normed[h][1] = pack_bf16x2(o.z * gn[s4].z, o.w * gn[s4].w);
-                        if (g.next_gain) {
-                            sq[t] += o.x * o.x;
-                            sq[t] += o.y * o.y;
-                            sq[t] += o.z * o.z;
-                            sq[t] += o.w * o.w;
-                        }
+                        if (g.next_gain) sq[t] = add_squares(sq[t], o.x, o.y, o.z, o.w);
                     }
                     if (g.next_gain) {
                         const int n = strip_of<EPI>(nb, wn, 4 * half + s2 + (quad & 1), g.N) * 16 + (quad & 2) * 4;
@@ -382,39 +377,26 @@ prefill_gemm(PrefillArgs a, GemmArgs g) {
             }
         }
         if (g.next_gain) {
-            const int parts = g.N / SQ_SPAN;
-#pragma unroll
-            for (int t = 0; t < WT; ++t) {
-                float v = sq[t];
-                v += lane_xor16(v);
-                v += lane_xor32(v);
-                const int m = m0 + (wm * WT + t) * 16 + lane % 16;
-                if (quad == 0 && m < a.M) g.out_sq[(size_t)m * parts + nb * (TN / SQ_SPAN) + wn] = v;
-            }
+            static_assert(WT == 4, "a row of 16 lanes to each of the wave's four tiles");
+            const float span = column_sums4(sq[0], sq[1], sq[2], sq[3]);  // the lanes of row q: tile q's rows
+            const int m = m0 + (wm * WT + quad) * 16 + lane % 16;
+            if (m < a.M) g.out_sq[(size_t)m * (g.N / SQ_SPAN) + nb * (TN / SQ_SPAN) + wn] = span;
         }
     } else if (EPI == EPI_SILU) {
         const int inner = g.N / 2;
         const float* scale = row_scale;
-        // silu(r g) (r u) for the row's scale r and the products g, u, as g u / ((1 + e) k) with
-        // e = 2^(-r log2(e) g) and k = 1 / r^2: the row's two constants once, then four VALU
-        // instructions and two transcendentals an output.
 #pragma unroll
         for (int t = 0; t < WT; ++t) {
             const int j = (wm * WT + t) * 16 + lane % 16;
             const int m = m0 + j;
             if (m >= a.M) continue;
-            const float rs = scale[j];
-            const float c = -rs * 1.4426950408889634f, k = __builtin_amdgcn_rcpf(rs * rs);
+            const SiluRow silu_row(scale[j]);
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
                 const int n = strip_of<EPI>(nb, wn, s, g.N) * 16 + quad * 4;
                 float v[4];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const float gp = acc[s][t][i], up = acc[s + 4][t][i];
-                    const float e = __builtin_amdgcn_exp2f(gp * c);
-                    v[i] = (gp * up) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, k, k));
-                }
+                for (int i = 0; i < 4; ++i) v[i] = silu_row(acc[s][t][i], acc[s + 4][t][i]);
                 uint2 packed = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
                 *reinterpret_cast<uint2*>(g.mlp + act_index(m, n, inner)) = packed;
             }
@@ -483,15 +465,8 @@ prefill_gemm(PrefillArgs a, GemmArgs g) {
                 if (rotate) {
                     const float2 co = *reinterpret_cast<const float2*>(t_cos + j * RS + e);
                     const float2 si = *reinterpret_cast<const float2*>(t_sin + j * RS + e);
-                    // As upstream: x cos + rotate_half(x) sin (rope_rows.comp:52-59), a pair
-                    // (x1, x2) to (x1 cos - x2 sin, x2 cos + x1 sin).
 #pragma unroll
-                    for (int k = 0; k < 2; ++k) {
-                        const float cs = k ? co.y : co.x, sn = k ? si.y : si.x;
-                        const float x1 = lo[k], x2 = hi[k];
-                        lo[k] = __builtin_fmaf(x1, cs, -(x2 * sn));
-                        hi[k] = __builtin_fmaf(x2, cs, x1 * sn);
-                    }
+                    for (int k = 0; k < 2; ++k) rotate_pair(lo[k], hi[k], k ? co.y : co.x, k ? si.y : si.x);
                 }
                 const int m = m0 + j;
                 if (head < H) {
@@ -1162,6 +1137,10 @@ hipError_t launch_prefill(const PrefillArgs& a, const PrefillLayer* layers, int 
                           const PrefillBuffers& b, hipStream_t stream, DispatchTimer* timer) {
     if (a.head_dim != 64 && a.head_dim != 128) return hipErrorInvalidValue;
     const int qkv_rows = (a.heads + 2 * a.kv_heads) * a.head_dim;
+    const bool by_rows = prefill_by_rows(a.M, a.hidden);
+    auto gemm = [&](int epi, int strip_rows, const GemmArgs& g) {
+        return launch_prefill_projection(a, epi, strip_rows, g, stream, timer);
+    };
     hipError_t e = hipSuccess;
     // Layer 0's input norm; each later norm's input (the rows times the gain, and their sums of
     // squares) comes from the projection before it, the rows' scales applied by the GEMM after.
@@ -1170,19 +1149,20 @@ hipError_t launch_prefill(const PrefillArgs& a, const PrefillLayer* layers, int 
     for (int l = 0; l < nlayers && e == hipSuccess; ++l) {
         const PrefillLayer& L = layers[l];
         GemmArgs qkv{L.qkv, b.normed, a.hidden, qkv_rows, nullptr, nullptr, nullptr, b.q, L.kv,
-                     l == 0 ? nullptr : b.row_sq, nullptr, nullptr, nullptr};
-        e = launch_prefill_gemm(a, EPI_QKV, QKV_ROWS, qkv, stream, timer);
+                     l == 0 || by_rows ? nullptr : b.row_sq, nullptr, nullptr, nullptr, nullptr};
+        if (l > 0 && by_rows) qkv.rows = b.h;
+        e = gemm(EPI_QKV, QKV_ROWS, qkv);
         if (e == hipSuccess) e = launch_prefill_attention(a, b.q, L.kv, b.attended, b.tiles, b.ntiles, stream, timer);
         GemmArgs o{L.o, b.attended, a.heads * a.head_dim, a.hidden, input, b.mid, nullptr, nullptr, nullptr,
-                   nullptr, L.post_norm, b.normed, b.row_sq};
-        if (e == hipSuccess) e = launch_prefill_gemm(a, EPI_RESIDUAL_IN, L.od_rows, o, stream, timer);
+                   nullptr, L.post_norm, b.normed, b.row_sq, nullptr};
+        if (e == hipSuccess) e = gemm(EPI_RESIDUAL_IN, L.od_rows, o);
         GemmArgs gu{L.gate_up, b.normed, a.hidden, 2 * a.inner, nullptr, nullptr, b.mlp, nullptr, nullptr,
-                    b.row_sq, nullptr, nullptr, nullptr};
-        if (e == hipSuccess) e = launch_prefill_gemm(a, EPI_SILU, QKV_ROWS, gu, stream, timer);
+                    b.row_sq, nullptr, nullptr, nullptr, nullptr};
+        if (e == hipSuccess) e = gemm(EPI_SILU, QKV_ROWS, gu);
         // The last layer's output goes to the final norm, which reads the f32 rows.
         GemmArgs down{L.down, b.mlp, a.inner, a.hidden, b.mid, b.h, nullptr, nullptr, nullptr,
-                      nullptr, l + 1 < nlayers ? layers[l + 1].input_norm : nullptr, b.normed, b.row_sq};
-        if (e == hipSuccess) e = launch_prefill_gemm(a, EPI_RESIDUAL, L.od_rows, down, stream, timer);
+                      nullptr, l + 1 < nlayers ? layers[l + 1].input_norm : nullptr, b.normed, b.row_sq, nullptr};
+        if (e == hipSuccess) e = gemm(EPI_RESIDUAL, L.od_rows, down);
         input = b.h;
     }
     if (e == hipSuccess) e = launch_prefill_norm(a, true, input, final_norm, nullptr, b.out, stream, timer);

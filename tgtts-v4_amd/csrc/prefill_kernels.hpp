@@ -5,8 +5,41 @@
 #include <stdint.h>
 
 #include "decode_kernels.hpp"
+#include "device.hpp"
 
 namespace tgx {
+
+// ---- arithmetic every prefill GEMM's epilogue shares, so that a row's bits are the same whichever
+// kernel its batch takes ----
+
+// The squares of a row's four columns added to `sum` in column order. A row's sum of squares is, over
+// each 128 columns (SQ_SPAN), an MFMA lane's 4 columns of each of the 8 strips in strip order from
+// zero, then the strip's four lanes as (l0 + l1) + (l2 + l3); and the spans in order.
+__device__ __forceinline__ float add_squares(float sum, float x, float y, float z, float w) {
+    return __builtin_fmaf(w, w, __builtin_fmaf(z, z, __builtin_fmaf(y, y, __builtin_fmaf(x, x, sum))));
+}
+// 1 / rms of a row of K columns from its sum of squares.
+__device__ __forceinline__ float rms_scale(float total, int K, float eps) { return 1.0f / sqrtf(total / (float)K + eps); }
+
+// silu(r g) (r u) for the row's scale r and the products g, u, as g u / ((1 + e) k) with
+// e = 2^(-r log2(e) g) and k = 1 / r^2: the row's two constants once, then four VALU instructions
+// and two transcendentals an output.
+struct SiluRow {
+    float c, k;
+    __device__ __forceinline__ explicit SiluRow(float rs) : c(-rs * 1.4426950408889634f), k(__builtin_amdgcn_rcpf(rs * rs)) {}
+    __device__ __forceinline__ float operator()(float gp, float up) const {
+        const float e = __builtin_amdgcn_exp2f(gp * c);
+        return (gp * up) * __builtin_amdgcn_rcpf(__builtin_fmaf(e, k, k));
+    }
+};
+
+// As upstream: x cos + rotate_half(x) sin (rope_rows.comp:52-59), a pair (x1, x2) to
+// (x1 cos - x2 sin, x2 cos + x1 sin).
+__device__ __forceinline__ void rotate_pair(float& x1, float& x2, float cs, float sn) {
+    const float a = x1, b = x2;
+    x1 = __builtin_fmaf(a, cs, -(b * sn));
+    x2 = __builtin_fmaf(b, cs, a * sn);
+}
 
 // A tile of up to 32 positions of one run for the attention: rows row0 .. row0 + count - 1 of
 // the prefill's tensors are positions pos0 .. pos0 + count - 1 of `slot`.
@@ -85,6 +118,9 @@ struct GemmArgs {
     const float* next_gain;
     uint16_t* out_n;
     float* out_sq;
+    // EPI_QKV of a short run (prefill_by_rows), in place of row_sq: the norm's input itself, f32
+    // [M_pad][K], whose sums of squares the GEMM takes.
+    const float* rows;
 };
 
 // The prefill's kernels one at a time, as launch_prefill launches them (the instance, grid and LDS
@@ -93,6 +129,15 @@ struct GemmArgs {
 // (layer 0's input norm into bf16 in fragment order, or the final norm into f32).
 hipError_t launch_prefill_gemm(const PrefillArgs& a, int epi, int strip_rows, const GemmArgs& g, hipStream_t stream,
                                DispatchTimer* timer);
+// The same GEMM by the kernel that suits its rows (prefill_short.hip, or launch_prefill_gemm's): the
+// same bits. Where prefill_by_rows, EPI_QKV takes g.rows and not g.row_sq, and EPI_RESIDUAL writes no
+// out_sq.
+hipError_t launch_prefill_projection(const PrefillArgs& a, int epi, int strip_rows, const GemmArgs& g, hipStream_t stream,
+                                     DispatchTimer* timer);
+// The line: q/k/v and down_proj by rows take 22.1 us a layer at 256 rows of hidden 1024 where the ring
+// takes 26.7 (16 and 33 at 128 rows of 2048: 34.4 and 45), at 512 rows 29.5 and 26.7.
+constexpr int PREFILL_ROWS_WORK = 256 * 1024;
+constexpr bool prefill_by_rows(int M, int hidden) { return (long long)M * hidden <= PREFILL_ROWS_WORK; }
 hipError_t launch_prefill_attention(const PrefillArgs& a, const uint16_t* q, const uint16_t* kv, uint16_t* attended,
                                     const PrefillTile* tiles, int ntiles, hipStream_t stream, DispatchTimer* timer);
 hipError_t launch_prefill_norm(const PrefillArgs& a, bool final, const float* x, const float* gain, uint16_t* out_bf16,
