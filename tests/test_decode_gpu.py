@@ -419,3 +419,48 @@ def test_rows_set_again_before_a_step_run_as_last_set(ctx):
         assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"step {t}"
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("head_dim,line", [(64, 1152), (128, 512)])
+def test_a_row_far_into_its_cache_gives_its_bits_among_many(ctx, head_dim, line):
+    """A step of few rows with one past decode_far positions takes its attention in chains, a
+    workgroup to each; one of more than 64 (row, KV head) groups takes it in one workgroup a group.
+    Rows around the line, with fewer than eight turns of 32 positions, with whole rounds of turns in
+    flight and a turn more or less: alone as among 33 rows, exactly; and a launch that moves a row
+    over the line as single steps."""
+    import tgx
+    from tgx.synth import StackSpec
+
+    wide = dict(hidden=2048, inner=6144) if head_dim == 128 else {}
+    spec = StackSpec(layers=2, dtype="bf16", head_dim=head_dim, **wide)
+    positions = [line - 2, line - 1, line, 1215, 1216, 1247, 1248, 2047, 2048, 2591]
+    others = [0, 31, 32, 200, 255, 256, 300, 511, 700] + [40 + 7 * k for k in range(14)]
+    at = positions + others
+    assert len(at) * spec.kv_heads > 64
+    dec = make_decoder(ctx, spec, 2816, rows=len(at), slots=len(at))
+    x = inputs(spec, sum(at) + len(at))
+    dec.prefill_runs([(r, 0, n) for r, n in enumerate(at) if n], x[: sum(at)])
+    last = x[sum(at) :]
+    among = dec.step_rows([tgx.Row(n, r) for r, n in enumerate(at)], last)
+    few = [None] * len(at)
+    for r, n in enumerate(positions):
+        print(f"[decode] position {n} alone, head_dim {head_dim}", flush=True)
+        few[r] = tgx.Row(n, r)
+        got = dec.step_rows(few, last)
+        few[r] = None
+        np.testing.assert_array_equal(got[r], among[r])
+    # Three steps over the line from one launch, against single steps.
+    few[0], few[12] = tgx.Row(line - 2, 0), tgx.Row(at[12], 12)
+    for t in range(3):
+        rows = [None] * len(at)
+        rows[0], rows[12] = tgx.Row(line - 2 + t, 0), tgx.Row(at[12] + t, 12)
+        single = dec.step_rows(rows, last)
+    dec.set_rows(few, last)
+    dec.launch(3, advance=True)
+    dec.wait()
+    dec.set_rows([None if r is None else tgx.Row(r.position + 2, r.slot) for r in few], last)
+    dec.start()
+    dec.wait()
+    got = dec.output()
+    for r in (0, 12):
+        np.testing.assert_array_equal(got[r], single[r])

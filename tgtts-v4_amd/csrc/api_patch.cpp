@@ -226,10 +226,7 @@ tgx_status tgx_patch_launch(tgx_lm_side* side, tgx_sampler* sampler, int times) 
         TGX_TRY(sampler_wait(s));
     }
     hipStream_t st = l->ctx->stream;
-    TGX_TRY(hold_ahead(l->base, times, 1));
-    TGX_TRY(hold_ahead(l->residual, times, 1));
-    TGX_TRY(sync_slots(l->base));
-    TGX_TRY(sync_slots(l->residual));
+    TGX_TRY(lm_side_hold_ahead(l, times, 1));
     const size_t mu_bytes = (size_t)l->rows * 2 * l->dit * 4;
     TGX_HIP(hipEventRecord(l->ev_start, st));
     for (int i = 0; i < times; ++i) {

@@ -21,6 +21,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 namespace tgx {
 
 namespace {
@@ -594,6 +596,156 @@ __global__ void __launch_bounds__(ATTN_THREADS) attention_decode(DecodeArgs a, L
 }
 
 // ---------------------------------------------------------------------------------------------
+// attention_chains and attention_join: attention_decode for a batch with a row far into its cache
+// (decode_far). One workgroup reads a row's whole cache there, at no more than one CU's rate (145 GB/s)
+// and two turns to a round trip. attention_chains gives each of its eight waves' chains of turns a
+// workgroup of its own (chain, KV head, row), a wave with DEPTH turns in flight, the next turn's scores
+// beside a turn's softmax, and leaves the chain's m, l and o; attention_join joins a row's eight in
+// order. Every turn, chain and join is attention_decode's arithmetic in its order: the same bits. What
+// bounds a chain is its serial softmax, 0.28 us a turn (DEPTH 4 and 6 alike). us a layer at head_dim
+// 64, two rows of 5003 and 12007 positions: 54.0 -> 14.3 + 4.0; one of 1200: 9.4 -> 4.2 + 4.0; at 128,
+// three of 12000: 106 -> 24 + 4.
+// A chain's state for its group's heads: m [16], l [16], then o [group][D], in f32.
+__host__ __device__ constexpr size_t chain_floats(int group, int head_dim) { return 32 + (size_t)group * head_dim; }
+
+// At head_dim 128 the turns in flight take more registers than two waves to a SIMD leave.
+template <int D>
+__global__ void __launch_bounds__(WAVE) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1))) attention_chains(DecodeArgs a, LayerArgs l) {
+    constexpr int TURN = attention_turn(D), DEPTH = 4;
+    constexpr int PT = TURN / 16, KS = PT / 2, DT = D / 16, DS = D / 32;
+    constexpr int KF = PT * DS, VF = DT * KS;
+    constexpr int BREGS = attention_capacity(D) / (ATTN_WAVES * WAVE * TURN);
+    constexpr int TILE = kv_tile(D);
+    const int w = blockIdx.x, kv = blockIdx.y, b = blockIdx.z, lane = threadIdx.x;
+    const int H = a.heads, KV = a.kv_heads, group = H / KV;
+    const int h = lane % 16;
+    const uint32_t pos = a.positions[b];
+    uint32_t turn_block[BREGS];
+#pragma unroll
+    for (int r = 0; r < BREGS; ++r)
+        turn_block[r] = a.row_table[(uint32_t)b * (uint32_t)a.max_blocks +
+                                    (uint32_t)min((w + ATTN_WAVES * (lane + WAVE * r)) * TURN / BLOCK_TOKENS, a.max_blocks - 1)];
+    uint4 qf[DS];
+#pragma unroll
+    for (int ds = 0; ds < DS; ++ds) qf[ds] = load16(l.q + ((size_t)b * H + kv * group + min(h, group - 1)) * D + ds * 32 + (lane / 16) * 8);
+    all_issued();
+    if (pos >= (uint32_t)a.capacity) return;  // a spare row
+    const int turns = (int)(pos / TURN) + 1;
+    const int count = turns > w ? (turns - 1 - w) / ATTN_WAVES + 1 : 0;  // this chain's
+    const int last = max(count - 1, 0);
+    static_assert(KS == 1 && BREGS <= 2, "a turn is half a block, and a chain has 128 turns at most");
+    auto block_of_turn = [&](int j) __attribute__((always_inline)) {
+        const int lo = __builtin_amdgcn_readlane((int)turn_block[0], j % WAVE);
+        if constexpr (BREGS == 1) return (uint32_t)lo;
+        const int hi = __builtin_amdgcn_readlane((int)turn_block[BREGS - 1], j % WAVE);
+        return (uint32_t)(j < WAVE ? lo : hi);
+    };
+    // Turn j's keys and values (attention_decode's fetch): every turn of a chain takes the same half of
+    // its block. Past the chain's last turn the last again.
+    const size_t stride = (size_t)KV * 2 * TILE;
+    const uint16_t* pool = l.kv + (size_t)kv * 2 * TILE + (w % 2) * KF * 512;  // uniform, as every turn's block
+    const int vat = TILE + (w % 2) * (512 - KF * 512);
+    uint4 kf[DEPTH][KF], vf[DEPTH][VF];
+    auto fetch = [&](int j, uint4 (&k)[KF], uint4 (&v)[VF]) __attribute__((always_inline)) {
+        const uint32_t blk = block_of_turn(min(j, last));
+        const uint16_t* at = pool + (blk < (uint32_t)a.nblocks ? blk : 0u) * stride;
+        const uint16_t* vt = at + vat;
+        // A uniform address plus the lane's 32-bit offset, no 64-bit adds to a lane.
+        auto load = [&](const uint16_t* p) __attribute__((always_inline)) {
+            return *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(p) + (uint32_t)lane * 16u);
+        };
+#pragma unroll
+        for (int i = 0; i < KF; ++i) k[i] = load(at + i * 512);
+#pragma unroll
+        for (int i = 0; i < VF; ++i) v[i] = load(vt + i * 1024);
+    };
+    OnlineSoftmax<PT, DT> sm;
+    const float scale_log2 = log2_scale(a.scale);
+    auto scores = [&](const uint4 (&k)[KF], f32x4 (&s)[PT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt) {
+            s[pt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int ds = 0; ds < DS; ++ds) s[pt] = mfma16(k[pt * DS + ds], qf[ds], s[pt]);
+        }
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        fetch(d, kf[d], vf[d]);
+        all_issued();
+    }
+    // Turn j's softmax and value products beside the next turn's scores.
+    f32x4 now[PT], next[PT];
+    scores(kf[0], now);
+    auto move_on = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt) now[pt] = next[pt];
+    };
+    int j = 0;
+    // Whole rounds while turns are left past them: none of these holds the row's position.
+    for (; j + DEPTH < count; j += DEPTH)
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) {
+            scores(kf[(d + 1) % DEPTH], next);
+            sm.template block<false>(now, vf[d], (uint32_t)(w + ATTN_WAVES * (j + d)) * TURN, pos, pos, scale_log2);
+            fetch(j + d + DEPTH, kf[d], vf[d]);
+            move_on();
+            all_issued();
+        }
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        if (j + d >= count) break;
+        if (d + 1 < DEPTH) scores(kf[(d + 1) % DEPTH], next);
+        const uint32_t p0 = (uint32_t)(w + ATTN_WAVES * (j + d)) * TURN;
+        if (p0 + TURN - 1 <= pos)
+            sm.template block<false>(now, vf[d], p0, pos, pos, scale_log2);
+        else
+            sm.template block<true>(now, vf[d], p0, pos, pos, scale_log2);
+        move_on();
+    }
+    float* state = l.chains + (((size_t)b * KV + kv) * ATTN_WAVES + w) * chain_floats(group, D);
+    if (lane < 16) {
+        state[h] = sm.m;
+        state[16 + h] = sm.l;
+    }
+    if (h < group) {
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+            *reinterpret_cast<float4*>(state + 32 + h * D + dt * 16 + (lane / 16) * 4) = make_float4(sm.o[dt][0], sm.o[dt][1], sm.o[dt][2], sm.o[dt][3]);
+    }
+}
+
+// Workgroup (KV head, row), a thread to an output.
+__global__ void __launch_bounds__(ATTN_THREADS) attention_join(DecodeArgs a, LayerArgs l) {
+    const int kv = blockIdx.x, b = blockIdx.y;
+    const int KV = a.kv_heads, group = a.heads / KV, D = a.head_dim;
+    const size_t each = chain_floats(group, D);
+    const float* state = l.chains + ((size_t)b * KV + kv) * ATTN_WAVES * each;
+    if (a.positions[b] >= (uint32_t)a.capacity) return;  // a spare row
+    for (int idx = threadIdx.x; idx < group * D; idx += ATTN_THREADS) {
+        const int hh = idx / D;
+        float m[ATTN_WAVES], sums[ATTN_WAVES], o[ATTN_WAVES];
+#pragma unroll
+        for (int j = 0; j < ATTN_WAVES; ++j) {
+            m[j] = state[j * each + hh];
+            sums[j] = state[j * each + 16 + hh];
+            o[j] = state[j * each + 32 + idx];
+        }
+        float M = -INFINITY;
+#pragma unroll
+        for (int j = 0; j < ATTN_WAVES; ++j) M = fmaxf(M, m[j]);
+        float L = 0.f, O = 0.f;
+#pragma unroll
+        for (int j = 0; j < ATTN_WAVES; ++j) {
+            const float f = sums[j] > 0.f ? __builtin_amdgcn_exp2f(m[j] - M) : 0.f;
+            L += sums[j] * f;
+            O += o[j] * f;
+        }
+        l.attended[operand_index(b, kv * group * D + idx, a.rows)] = (uint16_t)bf16_bits(O / L);
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
 // final_rmsnorm: the final norm, a wave to a row, for hidden = CH 1024; with `advance`, moves each
 // placed row on by one position once the step is done with it.
 template <int CH>
@@ -699,6 +851,10 @@ KernelLaunch attention_launch(const DecodeArgs& a) {
     return k;
 }
 
+size_t decode_chain_floats(const DecodeArgs& a) {
+    return (size_t)a.rows * a.kv_heads * ATTN_WAVES * chain_floats(a.heads / a.kv_heads, a.head_dim);
+}
+
 KernelLaunch residual_launch(const DecodeArgs& a, const ResidualArgs& r) {
     const int chunks = r.K / CHUNK_COLS;
     KernelLaunch k;
@@ -750,7 +906,19 @@ hipError_t launch_decode_layer(const DecodeArgs& a, const LayerArgs& l, const Re
     // The squares o_proj and down_proj leave span their strips' rows: 16 columns at 16-row strips.
     const bool wide = o.R == SQ_WIDE_COLS;
     hipError_t e = dispatch_launch("gemv_qkv_rope", qkv_launch(a, l.xn != nullptr, wide), layer_params, stream, timer);
-    if (e == hipSuccess) e = dispatch_launch("attention_decode", attention_launch(a), layer_params, stream, timer);
+    if (e == hipSuccess && l.chains) {
+        KernelLaunch k;
+        k.func = a.head_dim == 128 ? (const void*)attention_chains<128> : (const void*)attention_chains<64>;
+        k.grid = dim3(ATTN_WAVES, a.kv_heads, a.rows);
+        k.block = dim3(WAVE);
+        e = dispatch_launch("attention_chains", k, layer_params, stream, timer);
+        k.func = (const void*)attention_join;
+        k.grid = dim3(a.kv_heads, a.rows);
+        k.block = dim3(ATTN_THREADS);
+        if (e == hipSuccess) e = dispatch_launch("attention_join", k, layer_params, stream, timer);
+    } else if (e == hipSuccess) {
+        e = dispatch_launch("attention_decode", attention_launch(a), layer_params, stream, timer);
+    }
     const KernelLaunch ko = residual_launch(a, o), kd = residual_launch(a, down);
     if (!ko.func || !kd.func) return hipErrorInvalidValue;
     void* o_params[] = {&aa, &oo};

@@ -43,6 +43,9 @@ struct LayerArgs {
     uint16_t* q;              // [rows][heads][head_dim] bf16
     uint16_t* kv;             // the layer's cache pool: [blocks][kv_heads][key tile, value tile]
     uint16_t* attended;       // [rows][heads head_dim] bf16
+    // With a row past decode_far positions: the attention's chains' states (decode_chain_floats), the
+    // attention then two dispatches (attention_chains, attention_join); else null, and one.
+    float* chains;
     const uint16_t* mid_n;    // o_proj's output times post_norm in bf16 [rows][hidden]
     const float* mid_sq;      // [rows][hidden / 4], or [rows][hidden / 16] (wide)
     const uint16_t* gate_up;  // tiled bf16 [2 inner][hidden]
@@ -86,6 +89,15 @@ int decode_max_k();
 int decode_max_hidden();
 // The longest capacity the attention takes at a head width: a lane to each turn a wave takes.
 int decode_max_capacity(int head_dim);
+// The positions past which a row makes its step take the attention in chains (attention_chains, then
+// attention_join: a dispatch more a layer), for a batch of `groups` placed rows times KV heads. us a
+// step of 24 layers one way and the other: one row at 1000 positions 666 and 672, at 1200 710 and
+// 680, at 3000 898 and 727; 16 rows at 1200 757 and 744; four layers at head_dim 128, 8 rows at 500
+// 262 and 254. Past 64 groups the one workgroup each already fills the chip: 64 rows at 2100 999 and
+// 998, at 4000 1292 and 1301, up to 8000 1718 and 1451.
+constexpr uint32_t decode_far(int groups, int head_dim) { return groups > 64 ? 4096 : head_dim == 64 ? 1152 : 512; }
+constexpr uint32_t DECODE_FAR_LEAST = 512;
+size_t decode_chain_floats(const DecodeArgs& a);
 size_t decode_attention_lds(int heads, int kv_heads, int head_dim);
 // Lets the attention take up to `device_lds` bytes of LDS per workgroup.
 hipError_t decode_prepare(size_t device_lds);

@@ -353,10 +353,7 @@ tgx_status patch_step_launch(PatchStep* p, int times, int advance) {
     TGX_TRY(sampler_prepare(s));
     if (s->exec_dirty) TGX_TRY(sampler_record(s));
     hipStream_t st = l->ctx->stream;
-    TGX_TRY(hold_ahead(l->base, times, advance));
-    TGX_TRY(hold_ahead(l->residual, times, advance));
-    TGX_TRY(sync_slots(l->base));
-    TGX_TRY(sync_slots(l->residual));
+    TGX_TRY(lm_side_hold_ahead(l, times, advance));
     const size_t mu_bytes = (size_t)l->rows * 2 * l->dit * 4;
     TGX_HIP(hipEventRecord(p->ev_start, st));
     for (int i = 0; i < times; ++i) {

@@ -93,9 +93,11 @@ tgx_status side_record(LmSide* s, int advance, hipGraphExec_t* exec) {
     return TGX_OK;
 }
 
-// The program of s->rows rows as the current one, recorded if it has not been.
+// The program of s->rows rows, and of the attention each LM's next step takes (Decoder::far), as the
+// current one, recorded if it has not been.
 tgx_status side_program(LmSide* s) {
-    auto it = s->programs.find(s->rows);
+    const int key = s->rows * 4 + (s->base->far ? 2 : 0) + (s->residual->far ? 1 : 0);
+    auto it = s->programs.find(key);
     if (it == s->programs.end()) {
         RowProgram p;
         tgx_status st = side_record(s, 0, &p.exec);
@@ -105,7 +107,7 @@ tgx_status side_program(LmSide* s) {
             return st;
         }
         p.dispatches = s->dispatches;
-        it = s->programs.emplace(s->rows, p).first;
+        it = s->programs.emplace(key, p).first;
     }
     s->exec = it->second.exec;
     s->advance_exec = it->second.advance;
@@ -290,15 +292,20 @@ tgx_status lm_side_set_rows(LmSide* s, const tgx_row* rows, int nrows, const flo
     return TGX_OK;
 }
 
+tgx_status lm_side_hold_ahead(LmSide* s, int times, int advance) {
+    TGX_TRY(hold_ahead(s->base, times, advance));
+    TGX_TRY(hold_ahead(s->residual, times, advance));
+    TGX_TRY(side_program(s));
+    TGX_TRY(sync_slots(s->base));
+    return sync_slots(s->residual);
+}
+
 tgx_status lm_side_launch(LmSide* s, int times, int advance) {
     if (!s) return fail(TGX_E_ARG, "null LM side");
     if (s->pending || s->base->pending || s->residual->pending) return fail(TGX_E_BUSY, "a step is under way");
     if (times <= 0) return fail(TGX_E_ARG, "times");
     hipStream_t st = s->ctx->stream;
-    TGX_TRY(hold_ahead(s->base, times, advance));
-    TGX_TRY(hold_ahead(s->residual, times, advance));
-    TGX_TRY(sync_slots(s->base));
-    TGX_TRY(sync_slots(s->residual));
+    TGX_TRY(lm_side_hold_ahead(s, times, advance));
     TGX_HIP(hipEventRecord(s->ev_start, st));
     for (int i = 0; i < times; ++i) {
         if (s->use_graph) {

@@ -143,7 +143,7 @@ struct LmSide {
     Linear enc_to_lm, fsq_in, fsq_out, fusion, lm_to_dit, res_to_dit, stop_proj, stop_head;
     float *enc = nullptr, *levels_out = nullptr, *lm_hidden = nullptr, *stop_hidden = nullptr;
     float *mu = nullptr, *stop_logits = nullptr;
-    std::map<int, RowProgram> programs;
+    std::map<int, RowProgram> programs;  // by rows and the LMs' `far` (side_program)
     hipGraphExec_t exec = nullptr, advance_exec = nullptr;  // the current program's
     int dispatches = 0;
     hipEvent_t ev_start = nullptr, ev_end = nullptr;
@@ -163,6 +163,8 @@ std::vector<LmHead> lm_side_heads();
 tgx_status lm_side_set_rows(LmSide* s, const tgx_row* rows, int nrows, const float* enc);
 // The program of `rows` rows for both LMs and the heads (decoder_use_rows).
 tgx_status lm_side_use_rows(LmSide* s, int rows);
+// hold_ahead for both LMs, their tables on the device and the program of the steps' rows and reach.
+tgx_status lm_side_hold_ahead(LmSide* s, int times, int advance);
 tgx_status lm_side_launch(LmSide* s, int times, int advance);
 tgx_status lm_side_wait(LmSide* s);
 tgx_status lm_side_read(LmSide* s, const char* tensor, float* out, size_t count);

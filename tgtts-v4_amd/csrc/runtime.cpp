@@ -280,6 +280,7 @@ LayerArgs Decoder::layer_args(int l) const {
     la.q = q;
     la.kv = kv + (size_t)l * nblocks * shape.kv_heads * 2 * kv_tile(shape.head_dim);
     la.attended = attended;
+    la.chains = far ? chains : nullptr;
     la.mid_n = xn_b;
     la.mid_sq = sq_b;
     la.gate_up = layers[l].gate_up;
@@ -342,7 +343,7 @@ tgx_status alloc(Decoder* d, T** out, size_t count, bool zero = true) {
 }
 
 // The step's dispatches on the context's stream, in order (decode_batch_graph's ops,
-// decode.rs:630-723): five a layer, then the final norm.
+// decode.rs:630-723): five a layer (six when far), then the final norm.
 hipError_t enqueue_step(Decoder* d, int advance, DispatchTimer* timer, int* dispatches) {
     hipStream_t s = d->ctx->stream;
     const DecodeArgs a = d->args();
@@ -351,7 +352,7 @@ hipError_t enqueue_step(Decoder* d, int advance, DispatchTimer* timer, int* disp
     for (int l = 0; l < d->shape.layers && err == hipSuccess; ++l) {
         // layer 0 reads x_in, which stays as written
         err = launch_decode_layer(a, d->layer_args(l), d->o_args(l), d->down_args(l), s, timer);
-        n += 5;
+        n += d->far ? 6 : 5;
     }
     const float* x = d->shape.layers > 0 ? d->h_a : d->x_in;
     if (err == hipSuccess) {
@@ -383,9 +384,10 @@ tgx_status record(Decoder* d, int advance, hipGraphExec_t* exec) {
     return TGX_OK;
 }
 
-// The program of d->rows rows as the current one, recorded if it has not been.
+}  // namespace
+
 tgx_status use_program(Decoder* d) {
-    auto it = d->programs.find(d->rows);
+    auto it = d->programs.find({d->rows, d->far});
     if (it == d->programs.end()) {
         Decoder::Program p;
         tgx_status st = record(d, 0, &p.step);
@@ -395,13 +397,15 @@ tgx_status use_program(Decoder* d) {
             return st;
         }
         p.dispatches = d->dispatches;
-        it = d->programs.emplace(d->rows, p).first;
+        it = d->programs.emplace(std::make_pair(d->rows, d->far), p).first;
     }
     d->step_exec = it->second.step;
     d->advance_exec = it->second.advance;
     d->dispatches = it->second.dispatches;
     return TGX_OK;
 }
+
+namespace {
 
 tgx_status create_inner(Decoder* d, const tgx_batch* batch) {
     const Shape& s = d->shape;
@@ -439,6 +443,7 @@ tgx_status create_inner(Decoder* d, const tgx_batch* batch) {
     TGX_TRY(alloc(d, &d->out, (size_t)R * h));
     TGX_TRY(alloc(d, &d->q, (size_t)R * H * D));
     TGX_TRY(alloc(d, &d->attended, (size_t)R * H * D));
+    if ((uint32_t)s.capacity > DECODE_FAR_LEAST) TGX_TRY(alloc(d, &d->chains, decode_chain_floats(d->args())));
     TGX_TRY(alloc(d, &d->mlp, (size_t)R * I));
     TGX_TRY(alloc(d, &d->kv, (size_t)s.layers * d->nblocks * KV * 2 * kv_tile(D)));
     TGX_TRY(alloc(d, &d->positions, (size_t)R));
@@ -529,6 +534,8 @@ tgx_status hold_ahead(Decoder* d, int times, int advance) {
     // times - 1 after it too: its slot must hold blocks for all of them (decode.rs:198-227 refuses
     // a placement past the cache on the host; here the blocks are held, the capacity refused).
     const uint64_t reach = advance ? (uint64_t)times : 1;
+    uint64_t farthest = 0;
+    int groups = 0;
     for (int b = 0; b < d->rows; ++b) {
         const uint32_t pos = d->placement_host[b];
         if (pos == TGX_SPARE) continue;
@@ -536,7 +543,10 @@ tgx_status hold_ahead(Decoder* d, int times, int advance) {
             return fail(TGX_E_SHAPE, "row " + std::to_string(b) + " at position " + std::to_string(pos) + " run " +
                                          std::to_string(reach) + " steps on passes a capacity of " + std::to_string(d->shape.capacity));
         TGX_TRY(hold_slot(d, d->placement_host[d->rows + b], (uint32_t)(pos + reach)));
+        farthest = std::max(farthest, (uint64_t)pos + reach);
+        groups += d->shape.kv_heads;
     }
+    d->far = farthest > decode_far(groups, d->shape.head_dim);
     return TGX_OK;
 }
 
@@ -796,10 +806,13 @@ tgx_status decoder_use_rows(Decoder* d, int rows) {
         return fail(TGX_E_SHAPE, std::to_string(rows) + " rows in a batch of " + std::to_string(d->max_rows));
     if (rows == d->rows) return TGX_OK;
     const int before = d->rows;
+    const bool far = d->far;
     d->rows = rows;
+    d->far = false;  // until rows are placed
     tgx_status st = use_program(d);
     if (st != TGX_OK) {
         d->rows = before;  // the program it had stays
+        d->far = far;
         return st;
     }
     // Every row spare until placed again.
@@ -830,6 +843,7 @@ tgx_status decoder_start(Decoder* d) {
     if (d->pending) return fail(TGX_E_BUSY, "a step is under way");
     hipStream_t s = d->ctx->stream;
     TGX_TRY(hold_ahead(d, 1, 0));
+    TGX_TRY(use_program(d));
     TGX_TRY(sync_slots(d));
     TGX_HIP(hipEventRecord(d->ev_start, s));
     if (d->timed || !d->use_graph) {
@@ -892,6 +906,7 @@ tgx_status decoder_launch(Decoder* d, int times, int advance) {
     if (times <= 0) return fail(TGX_E_ARG, "times");
     hipStream_t s = d->ctx->stream;
     TGX_TRY(hold_ahead(d, times, advance));
+    TGX_TRY(use_program(d));
     TGX_TRY(sync_slots(d));
     TGX_HIP(hipEventRecord(d->ev_start, s));
     for (int i = 0; i < times; ++i) {

@@ -122,9 +122,13 @@ struct Decoder {
         hipGraphExec_t step = nullptr, advance = nullptr;
         int dispatches = 0;
     };
-    std::map<int, Program> programs;
+    std::map<std::pair<int, bool>, Program> programs;  // by rows, and whether far
     hipGraphExec_t step_exec = nullptr, advance_exec = nullptr;
     int dispatches = 0;
+    // Whether the next steps take their attention in chains (hold_ahead: a row past decode_far), and
+    // the chains' states.
+    bool far = false;
+    float* chains = nullptr;
     hipEvent_t ev_start = nullptr, ev_end = nullptr, ev_done = nullptr;
     bool pending = false;
     bool timed = false;  // launch dispatch by dispatch, each timed (Decoder::new's `timed`)
@@ -177,8 +181,10 @@ tgx_status hold_slot(Decoder* d, uint32_t slot, uint32_t positions);
 tgx_status sync_slots(Decoder* d);
 // Before `times` steps (each placed row moved on a position a step with `advance`): holds every
 // placed row's blocks up to the last position the steps write, refusing (TGX_E_SHAPE) a row the
-// steps would take past the capacity, or a pool that runs out.
+// steps would take past the capacity, or a pool that runs out; and sets `far` for the steps.
 tgx_status hold_ahead(Decoder* d, int times, int advance);
+// The program of the decoder's rows and `far` as the current one, recorded if it has not been.
+tgx_status use_program(Decoder* d);
 // The host's copy of the placement moved on as an advancing step moves the rows on the device.
 void moved_on(Decoder* d, int times);
 tgx_status prefill_runs(Decoder* d, const tgx_run* runs, int nruns, const float* x, float* out);
