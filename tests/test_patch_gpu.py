@@ -468,3 +468,50 @@ def test_fresh_patch_steps_beside_used_ones_give_a_warm_steps_bits_on_their_firs
         assert np.array_equal(alone[0].view(np.uint32), warm[0][pick].view(np.uint32)), f"fresh set {trial}: rows {pick}"
         close(parts, step)
         print(f"[patch] fresh set {trial}: first run bit for bit as the warm step's", flush=True)
+
+
+@pytest.mark.parametrize("feat,frames,rows", [(64, 4, (1, 3, 4, 12, 13)), (16, 1, (1, 8, 32, 33)), (48, 3, (2, 16, 17)), (32, 2, (1, 21, 22))])
+def test_an_encoder_of_any_rows_matches_the_oracle_and_gives_the_same_bits(ctx, feat, frames, rows):
+    """The local stack on both sides of its line at 64 tokens (o_proj and down_proj by local_gemm_sum
+    up to it, by the ring past it), at part-filled tiles, and the embedding at every count of frames
+    and of channels: each row against the oracle, and the same bits whatever its encoder's rows."""
+    import patch_oracle as po
+    import tgx
+    from tgx.patch import Encoder, PatchShape
+    from tgx.synth import encoder_weights
+
+    spec = _encoder_spec(layers=2)
+    w = encoder_weights(spec, feat)
+    shape = tgx.Shape(hidden=spec.hidden, inner=spec.inner, heads=spec.heads, kv_heads=spec.kv_heads,
+                      head_dim=spec.head_dim, layers=spec.layers, capacity=16, eps=spec.eps, rope_theta=spec.rope_theta)
+    patches = np.random.default_rng(15).standard_normal((max(rows), feat, frames)).astype(np.float32)
+    s = po.StackShape(hidden=spec.hidden, inner=spec.inner, heads=spec.heads, kv_heads=spec.kv_heads,
+                      layers=spec.layers, eps=spec.eps, rope_theta=spec.rope_theta)
+    want = po.encode(w, s, feat, frames, patches)
+    most = None
+    for n in sorted(rows, reverse=True):
+        print(f"[encoder] {n} rows of {frames} frames of {feat} channels", flush=True)
+        e = Encoder(ctx, shape, PatchShape(feat, frames, STEPS, n))
+        e.load_all(w)
+        got = e.encode(patches[:n])
+        e.close()
+        most = got if most is None else most
+        for r in range(n):
+            assert within(distance(got[r], want[r])), r
+        np.testing.assert_array_equal(got, most[:n])
+
+
+def test_samplers_around_64_tokens_give_a_request_the_same_bits(ctx):
+    """Two requests' 44 tokens go through the kernels for at most 64, three's 66 through the ring's."""
+    from tgx.synth import sampler_weights
+
+    spec = _dit_spec(layers=2)
+    w = sampler_weights(spec, FEAT)
+    mu, cond, noise, sampling = _inputs(3)
+    most = None
+    for n in (3, 2, 1):
+        s = _sampler(ctx, n, spec, w)
+        got = s.sample(mu[:n], cond[:n], noise[:n], sampling[:n])
+        s.close()
+        most = got if most is None else most
+        np.testing.assert_array_equal(got, most[:n])

@@ -127,10 +127,9 @@ tgx_status encoder_create(Context* ctx, const tgx_shape* stack, const tgx_patch_
     A(&e->x0, Mp * h);
     A(&e->x, Mp * h);
     A(&e->h, Mp * h);
-    A(&e->partial, (size_t)LOCAL_MAX_PARTS * Mp * h);
     A(&e->out, Mp * h);
     A(&e->normed, Mp * h);
-    A(&e->row_sq, Mp * (h / LOCAL_SQ_COLS));
+    A(&e->row_sq, local_sq_floats(Mp, h));
     A(&e->q, Mp * att);
     A(&e->k, Mp * KV * HEAD_DIM);
     A(&e->v, Mp * KV * HEAD_DIM);
@@ -201,12 +200,12 @@ hipError_t encoder_enqueue(Encoder* e, const float* patch, float* dst, int* disp
         layers[l] = LocalLayer{L.qkv, L.o, L.gate_up, L.down, L.input_norm, L.post_norm};
     }
     const LocalBuffers b{e->x0, e->x,        e->h,   e->normed,  e->row_sq, e->normed, e->row_sq,   e->q,
-                         e->k,  e->v,        e->attended, e->mlp, e->partial, e->out,  e->o_parts, e->down_parts};
+                         e->k,  e->v,        e->attended, e->mlp, e->out,  e->o_parts, e->down_parts};
     if (err == hipSuccess) err = launch_local_stack(a, layers.data(), e->shape.layers, e->final_norm, b, st, nullptr);
     // The learned token's output, the first of each sequence (encoder.rs:113-114).
     const size_t row = (size_t)e->shape.hidden * sizeof(float);
     if (err == hipSuccess) err = hipMemcpy2DAsync(dst, row, e->out, (size_t)e->T * row, row, e->rows, hipMemcpyDeviceToDevice, st);
-    if (dispatches) *dispatches = 1 + local_stack_dispatches(a, b, e->shape.layers);  // the embedding, the stack
+    if (dispatches) *dispatches = 1 + local_stack_dispatches(b, e->shape.layers);  // the embedding, the stack
     return err;
 }
 

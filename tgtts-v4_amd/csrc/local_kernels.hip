@@ -15,8 +15,8 @@
 //   local_attention every token of a sequence attends to every token of it, a wave to a
 //                   sequence and query head, both products on MFMA (local_attention.comp)
 //   local_add_norm  residual + the parts' sums in their order, then the next norm's input
-//                   (local_add_norm.comp, local_norm.comp): up to 64 tokens, and the first and
-//                   final norms
+//                   (local_add_norm.comp, local_norm.comp): the first and final norms, and behind
+//                   local_gemm's parts by name
 //   local_embed     a linear layer over a patch's frames into tokens, and tokens copied beside
 //                   them (local_embed.comp)
 //   dit_euler       out_proj's velocities, CFG-Zero* guidance and the Euler step (dit_euler.comp)
@@ -28,6 +28,8 @@
 #include "local_kernels.hpp"
 
 #include <math.h>
+
+#include <type_traits>
 
 #include "dispatch.hpp"
 
@@ -90,7 +92,43 @@ struct RowSq {
             p[i] = __builtin_bit_cast(float4, t);
         }
     }
+    __device__ float scale(int K, float eps) const { return row_scale_of(p, K, eps); }
 };
+
+// A row's sums of squares over each 16 columns (local_gemm_sum's), [tokens][K / 16]: the four lanes of
+// a column take a quarter of the row's SQ_PARTS spans each, four sums to a span, and pass the spans
+// round; added in the order RowSq's have.
+struct RowSqFine {
+    float4 p[SQ_PARTS / 4];
+    __device__ void load(const float* row_sq, int m) {
+        const int quad = threadIdx.x % WAVE / 16;
+#pragma unroll
+        for (int i = 0; i < SQ_PARTS / 4; ++i)
+            p[i] = *reinterpret_cast<const float4*>(row_sq + (size_t)m * (4 * SQ_PARTS) + (quad * (SQ_PARTS / 4) + i) * 4);
+    }
+    __device__ void settle() {
+        typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+        for (int i = 0; i < SQ_PARTS / 4; ++i) {
+            u32x4 t = __builtin_bit_cast(u32x4, p[i]);
+            asm volatile("" : "+v"(t));
+            p[i] = __builtin_bit_cast(float4, t);
+        }
+    }
+    __device__ float scale(int K, float eps) const {
+        float s[SQ_PARTS / 4];
+#pragma unroll
+        for (int i = 0; i < SQ_PARTS / 4; ++i) s[i] = (p[i].x + p[i].y) + (p[i].z + p[i].w);
+        float total = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < SQ_PARTS / 4; ++i) total += __shfl(s[i], threadIdx.x % 16 + 16 * q, WAVE);
+        return 1.0f / sqrtf(total / (float)K + eps);
+    }
+};
+template <bool FINE>
+using RowSquares = std::conditional_t<FINE, RowSqFine, RowSq>;
 
 // A wave's strips of W for work unit u: SW strips in a row, or for the gate/up projection (SW 2)
 // gate strip u and the same rows of up, N / 32 strips on.
@@ -227,8 +265,8 @@ struct WeightRing {
 // local_gemm_direct, for at most 64 tokens (M_pad = 16 TT): a workgroup of TT waves to a work unit
 // (SW strips of W), wave t against token tile t, both operands straight from memory into
 // registers, DEPTH k-blocks ahead (the waves read the same W; all but the first find it in cache).
-// Grid (units, 1, parts).
-template <int EPI, int SW, int TT, int KBP>
+// Grid (units, 1, parts). FINE: g.row_sq is over each 16 columns.
+template <int EPI, int SW, int TT, int KBP, bool FINE>
 __global__ void __launch_bounds__(TT * WAVE) local_gemm_direct(LocalArgs a, LocalGemm g) {
     constexpr int DEPTH = LG_INFLIGHT / (SW + 1) < KBP ? LG_INFLIGHT / (SW + 1) : KBP;
     const int t = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
@@ -237,7 +275,7 @@ __global__ void __launch_bounds__(TT * WAVE) local_gemm_direct(LocalArgs a, Loca
     local_strips<EPI, SW>(blockIdx.x, g.N, strip);
     // The lane's token's sums of squares go first, the GEMM's loads behind them.
     constexpr bool SCALED = EPI == LEPI_QKV || EPI == LEPI_SILU;
-    RowSq sq;
+    RowSquares<FINE> sq;
     if (SCALED) sq.load(g.row_sq, 16 * t + lane % 16);
     WeightRing<SW, KBP, DEPTH> w;
     w.start(g, strip, kb0, lane);
@@ -264,8 +302,62 @@ __global__ void __launch_bounds__(TT * WAVE) local_gemm_direct(LocalArgs a, Loca
         }
         all_issued();  // each k-block's refill stays where it is, DEPTH k-blocks ahead of its use
     }
-    const float rs[1] = {SCALED ? row_scale_of(sq.p, g.K, a.eps) : 1.f};
+    const float rs[1] = {SCALED ? sq.scale(g.K, a.eps) : 1.f};
     local_epilogue<EPI, SW, 1>(a, g, strip, 16 * t, acc, rs);
+}
+
+// local_gemm_sum, o_proj and down_proj for at most 64 tokens: a workgroup of P waves to a strip of W
+// and a token tile, wave p its part of K, both operands straight from memory as local_gemm_direct's;
+// the parts' sums through LDS, then wave 0 adds them in part order, the residual, and writes the
+// next norm's input and its sums of squares over the strip's 16 columns (RowSqFine). In one dispatch
+// what local_gemm_direct and local_add_norm take two for, the same bits: at these sizes a dispatch is
+// its launch and one trip to memory (22 tokens: 4.2 + 4.5 us -> 4.4, 72 times a one-request sample).
+// Grid (N / 16, M_pad / 16); a strip's tiles sit on one XCD.
+template <int KBP, int P>
+__global__ void __launch_bounds__(P * WAVE) local_gemm_sum(LocalArgs a, LocalGemm g) {
+    constexpr int DEPTH = LG_INFLIGHT / 2 < KBP ? LG_INFLIGHT / 2 : KBP;
+    __shared__ f32x4 red[P][WAVE];
+    const int p = threadIdx.x / WAVE, lane = threadIdx.x % WAVE, quad = lane / 16;
+    const int strip[1] = {(int)blockIdx.x};
+    const int m = blockIdx.y * 16 + lane % 16, n = strip[0] * 16 + quad * 4;
+    const float4 r = *reinterpret_cast<const float4*>(g.residual + (size_t)m * g.N + n);
+    const float4 gn = *reinterpret_cast<const float4*>((g.next_gain ? g.next_gain : g.residual) + n);
+    WeightRing<1, KBP, DEPTH> w;
+    w.start(g, strip, p * KBP, lane);
+    const uint16_t* xp = g.x + act_index(blockIdx.y * 16, p * KBP * 32, g.K) + lane * 8;
+    uint4 xf[DEPTH];
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+        w.fetch(d, d + 1);
+        xf[d] = load16(xp + d * 512);
+    }
+    all_issued();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < KBP; ++kb) {
+        acc = mfma16(w.wf[kb % DEPTH][0], xf[kb % DEPTH], acc);
+        if (kb + DEPTH < KBP) {
+            w.fetch(kb + DEPTH, kb + DEPTH + 1);
+            xf[kb % DEPTH] = load16(xp + (kb + DEPTH) * 512);
+        }
+        all_issued();
+    }
+    red[p][lane] = acc;
+    __syncthreads();
+    if (p) return;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < P; ++i) sum += red[i][lane];
+    const float4 v = make_float4(r.x + sum[0], r.y + sum[1], r.z + sum[2], r.w + sum[3]);
+    float s4 = squares4(v.x, v.y, v.z, v.w);
+    s4 += lane_xor16(s4);
+    s4 += lane_xor32(s4);
+    if (m >= a.M) return;
+    *reinterpret_cast<float4*>(g.sum + (size_t)m * g.N + n) = v;
+    if (!g.next_gain) return;
+    *reinterpret_cast<uint2*>(g.normed + act_index(m, n, g.N)) =
+        make_uint2(pack_bf16x2(v.x * gn.x, v.y * gn.y), pack_bf16x2(v.z * gn.z, v.w * gn.w));
+    if (quad == 0) g.sum_sq[(size_t)m * (4 * SQ_PARTS) + strip[0]] = s4;
 }
 
 // local_gemm_ring, for more tokens (M_pad a multiple of 16 TT): a workgroup of 4 waves to 16 TT
@@ -449,13 +541,19 @@ void local_gemm(const char* label, const LocalArgs& a, const LocalGemm& g, int u
                 DispatchTimer* timer) {
     if (a.M_pad <= 64) {
         const dim3 grid(units, 1, parts);
-        switch (a.M_pad / 16) {
-            case 1: dispatch(label, local_gemm_direct<EPI, SW, 1, KBP>, grid, dim3(WAVE), 0, stream, timer, a, g); break;
-            case 2: dispatch(label, local_gemm_direct<EPI, SW, 2, KBP>, grid, dim3(2 * WAVE), 0, stream, timer, a, g); break;
-            case 3: dispatch(label, local_gemm_direct<EPI, SW, 3, KBP>, grid, dim3(3 * WAVE), 0, stream, timer, a, g); break;
-            default: dispatch(label, local_gemm_direct<EPI, SW, 4, KBP>, grid, dim3(4 * WAVE), 0, stream, timer, a, g); break;
+        auto direct = [&](auto fine) {
+            constexpr bool FINE = decltype(fine)::value;
+            switch (a.M_pad / 16) {
+                case 1: dispatch(label, local_gemm_direct<EPI, SW, 1, KBP, FINE>, grid, dim3(WAVE), 0, stream, timer, a, g); break;
+                case 2: dispatch(label, local_gemm_direct<EPI, SW, 2, KBP, FINE>, grid, dim3(2 * WAVE), 0, stream, timer, a, g); break;
+                case 3: dispatch(label, local_gemm_direct<EPI, SW, 3, KBP, FINE>, grid, dim3(3 * WAVE), 0, stream, timer, a, g); break;
+                default: dispatch(label, local_gemm_direct<EPI, SW, 4, KBP, FINE>, grid, dim3(4 * WAVE), 0, stream, timer, a, g); break;
+            }
+        };
+        if constexpr (EPI != LEPI_PARTIAL) {
+            if (g.fine) return direct(std::true_type{});
         }
-        return;
+        return direct(std::false_type{});
     }
     // Eight token tiles a workgroup for gate/up where the tokens come in 128s (its W, 16 MiB at
     // the sampler's shape, is the most read); four otherwise.
@@ -469,6 +567,19 @@ void local_gemm(const char* label, const LocalArgs& a, const LocalGemm& g, int u
     if constexpr (EPI != LEPI_PARTIAL)
         dispatch(label, local_gemm_ring<EPI, SW, KBP, 1, 4>, dim3(units / 4, a.M_pad / 64), dim3(4 * WAVE), ring_lds(SW, 4), stream,
                  timer, a, g);
+}
+
+// o_proj and down_proj for at most 64 tokens, their parts added with the residual in one dispatch.
+void local_sum(const char* label, const LocalArgs& a, const LocalGemm& g, int kbp, int parts, hipStream_t stream, DispatchTimer* timer) {
+    const dim3 grid(g.N / 16, a.M_pad / 16), block(parts * WAVE);
+    if (kbp == 16 && parts == 2)
+        dispatch(label, local_gemm_sum<16, 2>, grid, block, 0, stream, timer, a, g);
+    else if (kbp == 32 && parts == 2)
+        dispatch(label, local_gemm_sum<32, 2>, grid, block, 0, stream, timer, a, g);
+    else if (kbp == 16 && parts == 4)
+        dispatch(label, local_gemm_sum<16, 4>, grid, block, 0, stream, timer, a, g);
+    else
+        dispatch(label, local_gemm_sum<32, 4>, grid, block, 0, stream, timer, a, g);
 }
 
 // o_proj and down_proj over more than 64 tokens: the ring with the parts added and the residual
@@ -637,7 +748,7 @@ __global__ void __launch_bounds__(256) local_add_norm(LocalArgs a, const float* 
 // sum_c W[n][c] frame_f[c] in channel order, written as token first + f of each of the row's sequences;
 // and wave t copied token t. W's 64 rows come in one piece, coalesced, and are handed to the lanes
 // through LDS: a lane reading its own row made each load 64 cache lines and left a row's 1024 columns
-// to four workgroups (one request 10.6 us -> 4.6; 16 requests 8.0 -> 4.9).
+// to four workgroups (one request 10.6 us -> 5.2; 16 requests 8.0 -> 4.9).
 constexpr int EMBED_MAX = 1024;     // channels x frames a row's patch may hold
 constexpr int EMBED_CHANNELS = 64;  // channels at most, a multiple of 4
 constexpr int EMBED_COPIES = 2;     // copied tokens at most
@@ -718,7 +829,8 @@ constexpr int EULER_STRIPS = 4;  // channels / 16 at most
 constexpr int EULER_K = 1024;    // the DiT's width
 constexpr int EULER_KB = EULER_K / 32 / EULER_WAVES;  // k-blocks to a wave
 
-template <int F>
+// FINE: e.row_sq is over each 16 columns.
+template <int F, bool FINE>
 __global__ void __launch_bounds__(EULER_THREADS) dit_euler(LocalArgs a, EulerArgs e) {
     constexpr int TOKENS = 2 * F, K = EULER_K, KB = K / 32;
     __shared__ f32x4 red[EULER_WAVES][EULER_STRIPS][WAVE];
@@ -733,7 +845,7 @@ __global__ void __launch_bounds__(EULER_THREADS) dit_euler(LocalArgs a, EulerArg
     const size_t token = (size_t)(row * 2 + tmc / F) * a.T + e.first + tmc % F;
     const float* src = e.x + token * K + (lane / 16) * 8;
     const float* gain = e.gain + (lane / 16) * 8;
-    RowSq sq;
+    RowSquares<FINE> sq;
     sq.load(e.row_sq, (int)token);
     float4 lo[EULER_KB], hi[EULER_KB], glo[EULER_KB], ghi[EULER_KB];
     uint4 wf[EULER_KB][EULER_STRIPS];
@@ -749,7 +861,7 @@ __global__ void __launch_bounds__(EULER_THREADS) dit_euler(LocalArgs a, EulerArg
             wf[j][s] = *reinterpret_cast<const uint4*>(e.w + weight_tile_index(min(s, strips - 1), kb, KB, 16) + lane * 8);
     }
     // The final norm: x / rms(x) g, its scale from the row's sums of squares.
-    const float scale = row_scale_of(sq.p, K, a.eps);
+    const float scale = sq.scale(K, a.eps);
     auto normed = [&](float4 v, float4 g4) { return make_float4(v.x * scale * g4.x, v.y * scale * g4.y, v.z * scale * g4.z, v.w * scale * g4.w); };
 #pragma unroll
     for (int j = 0; j < EULER_KB; ++j) {
@@ -869,10 +981,13 @@ hipError_t launch_local_add_norm(const LocalArgs& a, bool final, const float* pa
 
 hipError_t launch_local_add(const LocalArgs& a, const LocalGemm& g, int parts, hipStream_t stream, DispatchTimer* timer) {
     const int kbp = parts > 0 ? g.K / 32 / parts : 0;
-    if (a.M_pad <= 64 || a.M_pad != local_rows_padded(a.M) || (parts != 2 && parts != 4) || (kbp != 16 && kbp != 32) ||
+    if (g.fine != (a.M_pad <= 64) || a.M_pad != local_rows_padded(a.M) || (parts != 2 && parts != 4) || (kbp != 16 && kbp != 32) ||
         kbp * 32 * parts != g.K || g.N != a.hidden)
         return hipErrorInvalidValue;
-    local_gemm_add("local_add", a, g, kbp, parts, stream, timer);
+    if (g.fine)
+        local_sum("local_add", a, g, kbp, parts, stream, timer);
+    else
+        local_gemm_add("local_add", a, g, kbp, parts, stream, timer);
     return hipGetLastError();
 }
 
@@ -888,16 +1003,15 @@ hipError_t launch_local_stack(const LocalArgs& a, const LocalLayer* layers, int 
         return hipErrorInvalidValue;
     const int H = a.heads, KV = a.kv_heads;
     const int qkv_rows = (H + 2 * KV) * HEAD_DIM;
-    // Over more than 64 tokens o_proj and down_proj add their parts and the residual themselves
-    // (the ring GEMM); up to 64, their parts go out to `partial` for local_add_norm to add.
-    const bool ring = a.M_pad > 64;
+    // o_proj and down_proj add their parts and the residual themselves; up to 64 tokens they leave the
+    // next norm's sums of squares over each 16 columns.
+    const bool fine = local_fine_sums(a.M_pad);
     hipError_t e = hipSuccess;
     // The first layer's input norm, unless the embedding wrote it.
     if (!b.normed0) e = launch_local_add_norm(a, false, nullptr, 0, b.x0, nullptr, layers[0].input_norm, b.normed, b.row_sq, nullptr, stream, timer);
     for (int l = 0; l < nlayers && e == hipSuccess; ++l) {
         const LocalLayer& L = layers[l];
         const bool last = l + 1 == nlayers;
-        const float* input = l == 0 ? b.x0 : b.x;
         LocalGemm qkv{};
         qkv.w = L.qkv;
         qkv.x = l == 0 && b.normed0 ? b.normed0 : b.normed;
@@ -907,6 +1021,7 @@ hipError_t launch_local_stack(const LocalArgs& a, const LocalLayer* layers, int 
         qkv.k = b.k;
         qkv.v = b.v;
         qkv.row_sq = l == 0 && b.normed0 ? b.row_sq0 : b.row_sq;
+        qkv.fine = fine && l > 0;  // the embedding's and the first norm's are over LOCAL_SQ_COLS
         e = launch_local_qkv(a, qkv, stream, timer);
         if (e == hipSuccess) e = launch_local_attention(a, b.q, b.k, b.v, b.attended, stream, timer);
         LocalGemm o{};
@@ -914,19 +1029,13 @@ hipError_t launch_local_stack(const LocalArgs& a, const LocalLayer* layers, int 
         o.x = b.attended;
         o.K = H * HEAD_DIM;
         o.N = a.hidden;
-        if (ring) {
-            o.residual = input;
-            o.sum = b.h;
-            o.next_gain = L.post_norm;
-            o.normed = b.normed;
-            o.sum_sq = b.row_sq;
-            if (e == hipSuccess) e = launch_local_add(a, o, b.o_parts, stream, timer);
-        } else {
-            o.partial = b.partial;
-            if (e == hipSuccess) e = launch_local_partial(a, o, b.o_parts, stream, timer);
-            if (e == hipSuccess)
-                e = launch_local_add_norm(a, false, b.partial, b.o_parts, input, b.h, L.post_norm, b.normed, b.row_sq, nullptr, stream, timer);
-        }
+        o.residual = l == 0 ? b.x0 : b.x;
+        o.sum = b.h;
+        o.next_gain = L.post_norm;
+        o.normed = b.normed;
+        o.sum_sq = b.row_sq;
+        o.fine = fine;
+        if (e == hipSuccess) e = launch_local_add(a, o, b.o_parts, stream, timer);
         LocalGemm gu{};
         gu.w = L.gate_up;
         gu.x = b.normed;
@@ -934,40 +1043,29 @@ hipError_t launch_local_stack(const LocalArgs& a, const LocalLayer* layers, int 
         gu.N = 2 * a.inner;
         gu.mlp = b.mlp;
         gu.row_sq = b.row_sq;
+        gu.fine = fine;
         if (e == hipSuccess) e = launch_local_gate_up(a, gu, stream, timer);
         LocalGemm down{};
         down.w = L.down;
         down.x = b.mlp;
         down.K = a.inner;
         down.N = a.hidden;
+        down.residual = b.h;
+        down.sum = b.x;
         // After the last layer, with no `out`, x and its sums of squares for the reader to norm.
-        const float* next_gain = !last ? layers[l + 1].input_norm : b.out ? nullptr : final_norm;
-        if (ring) {
-            down.residual = b.h;
-            down.sum = b.x;
-            down.next_gain = next_gain;
-            down.normed = b.normed;
-            down.sum_sq = b.row_sq;
-            if (e == hipSuccess) e = launch_local_add(a, down, b.down_parts, stream, timer);
-            if (e == hipSuccess && last && b.out)
-                e = launch_local_add_norm(a, true, nullptr, 0, b.x, nullptr, final_norm, nullptr, nullptr, b.out, stream, timer);
-            continue;
-        }
-        down.partial = b.partial;
-        if (e == hipSuccess) e = launch_local_partial(a, down, b.down_parts, stream, timer);
-        if (e != hipSuccess) break;
-        if (next_gain)
-            e = launch_local_add_norm(a, false, b.partial, b.down_parts, b.h, b.x, next_gain, b.normed, b.row_sq, nullptr, stream, timer);
-        else
-            e = launch_local_add_norm(a, true, b.partial, b.down_parts, b.h, b.x, final_norm, nullptr, nullptr, b.out, stream, timer);
+        down.next_gain = !last ? layers[l + 1].input_norm : b.out ? nullptr : final_norm;
+        down.normed = b.normed;
+        down.sum_sq = b.row_sq;
+        down.fine = fine;
+        if (e == hipSuccess) e = launch_local_add(a, down, b.down_parts, stream, timer);
+        if (e == hipSuccess && last && b.out)
+            e = launch_local_add_norm(a, true, nullptr, 0, b.x, nullptr, final_norm, nullptr, nullptr, b.out, stream, timer);
     }
     return e;
 }
 
-int local_stack_dispatches(const LocalArgs& a, const LocalBuffers& b, int nlayers) {
-    const int norms = b.normed0 ? 0 : 1;
-    if (a.M_pad > 64) return norms + 5 * nlayers + (b.out ? 1 : 0);
-    return norms + 7 * nlayers;
+int local_stack_dispatches(const LocalBuffers& b, int nlayers) {
+    return (b.normed0 ? 0 : 1) + 5 * nlayers + (b.out ? 1 : 0);
 }
 
 bool local_supported(int hidden, int inner, int heads, int kv_heads, int o_parts, int down_parts) {
@@ -1009,13 +1107,18 @@ hipError_t launch_local_embed(const LocalArgs& a, const EmbedArgs& e, int rows, 
 hipError_t launch_dit_euler(const LocalArgs& a, const EulerArgs& e, int rows, hipStream_t stream, DispatchTimer* timer) {
     if (a.hidden != EULER_K) return hipErrorInvalidValue;
     const dim3 grid(rows), block(EULER_THREADS);
-    switch (e.frames) {
-        case 1: dispatch("dit_euler", dit_euler<1>, grid, block, 0, stream, timer, a, e); break;
-        case 2: dispatch("dit_euler", dit_euler<2>, grid, block, 0, stream, timer, a, e); break;
-        case 3: dispatch("dit_euler", dit_euler<3>, grid, block, 0, stream, timer, a, e); break;
-        case 4: dispatch("dit_euler", dit_euler<4>, grid, block, 0, stream, timer, a, e); break;
-        default: return hipErrorInvalidValue;
-    }
+    auto by_frames = [&](auto fine) {
+        constexpr bool FINE = decltype(fine)::value;
+        switch (e.frames) {
+            case 1: dispatch("dit_euler", dit_euler<1, FINE>, grid, block, 0, stream, timer, a, e); return hipSuccess;
+            case 2: dispatch("dit_euler", dit_euler<2, FINE>, grid, block, 0, stream, timer, a, e); return hipSuccess;
+            case 3: dispatch("dit_euler", dit_euler<3, FINE>, grid, block, 0, stream, timer, a, e); return hipSuccess;
+            case 4: dispatch("dit_euler", dit_euler<4, FINE>, grid, block, 0, stream, timer, a, e); return hipSuccess;
+            default: return hipErrorInvalidValue;
+        }
+    };
+    const hipError_t err = e.fine ? by_frames(std::true_type{}) : by_frames(std::false_type{});
+    if (err != hipSuccess) return err;
     return hipGetLastError();
 }
 

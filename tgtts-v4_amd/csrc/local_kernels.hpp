@@ -41,8 +41,8 @@ struct LocalBuffers {
     // contiguous KiB), so that a wave's load of one is one contiguous KiB.
     uint16_t* normed;    // bf16 [M_pad][hidden], fragment order: an RMSNorm's input times its gain, the rows' scales
                          // still to apply (the GEMM that reads it applies them)
-    float* row_sq;       // f32 [M_pad][hidden / LOCAL_SQ_COLS]: normed's rows' sums of squares, each
-                         // over LOCAL_SQ_COLS columns
+    float* row_sq;       // f32: normed's rows' sums of squares, each over LOCAL_SQ_COLS columns, or over 16
+                         // up to 64 tokens (local_fine_sums): local_sq_floats(M_pad, hidden)
     // The first layer's normed input and its sums of squares, as the embedding wrote them
     // (EmbedArgs::gain); null for the stack to norm x0 itself.
     const uint16_t* normed0;
@@ -50,7 +50,6 @@ struct LocalBuffers {
     uint16_t *q, *k, *v; // bf16 [M_pad][heads | kv_heads][64]
     uint16_t* attended;  // bf16 [M_pad][heads 64], fragment order
     uint16_t* mlp;       // bf16 [M_pad][inner], fragment order
-    float* partial;      // f32 [LOCAL_MAX_PARTS][M_pad][hidden]
     // f32 [M_pad][hidden]: the last layer's output after the final norm; null to leave the norm
     // to the stack's reader (x and row_sq then hold its input and sums of squares)
     float* out;
@@ -82,7 +81,7 @@ struct EmbedArgs {
 // final norm is taken here, for the tokens read.
 struct EulerArgs {
     const float* x;       // f32 [M_pad][hidden], the stack's last residual (before its final norm)
-    const float* row_sq;  // x's sums of squares, [M_pad][hidden / LOCAL_SQ_COLS]
+    const float* row_sq;  // x's sums of squares, [M_pad][hidden / LOCAL_SQ_COLS] (fine: / 16)
     const float* gain;    // the final norm's gain [hidden]
     const uint16_t* w;  // bf16 [channels][hidden] in 16-row MFMA tiles
     const float* bias;  // [channels]
@@ -90,6 +89,7 @@ struct EulerArgs {
     float* state;       // [rows][channels][frames]
     int channels, frames, first;
     float dt;
+    bool fine;
 };
 
 // What a local stack's projection writes beside its products (local_gemm_direct, local_gemm_ring):
@@ -108,19 +108,21 @@ struct LocalGemm {
     // LEPI_QKV, LEPI_SILU: X is an RMSNorm's input times its gain; row m's sums of squares
     // [M_pad][K / LOCAL_SQ_COLS] give the row's scale, applied to its sums.
     const float* row_sq;
-    // LEPI_ADD (local_gemm_ring): sum = residual + the parts' sums, and with next_gain, the next
+    // LEPI_ADD (local_gemm_ring, local_gemm_sum): sum = residual + the parts' sums, and with next_gain, the next
     // norm's input: normed = sum next_gain in bf16 and sum's sums of squares into sum_sq.
     const float* residual;
     float* sum;
     const float* next_gain;
     uint16_t* normed;
     float* sum_sq;
+    // row_sq and sum_sq are over each 16 columns, not LOCAL_SQ_COLS (up to 64 tokens).
+    bool fine;
 };
 
 // The local stack's kernels one at a time, as launch_local_stack launches them: q/k/v with RoPE
 // (its N the q/k/v rows), the attention within each sequence, o_proj's or down_proj's parts
 // (up to 64 tokens) and their sum with the residual and the next norm's input (or the final norm
-// into `out`), the same fused (past 64 tokens; 2 or 4 parts), and gate/up with SiLU.
+// into `out`), the same fused (2 or 4 parts; g.fine up to 64 tokens), and gate/up with SiLU.
 hipError_t launch_local_qkv(const LocalArgs& a, const LocalGemm& g, hipStream_t stream, DispatchTimer* timer);
 hipError_t launch_local_attention(const LocalArgs& a, const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* attended,
                                   hipStream_t stream, DispatchTimer* timer);
@@ -138,10 +140,17 @@ hipError_t local_prepare();
 bool local_supported(int hidden, int inner, int heads, int kv_heads, int o_parts, int down_parts);
 // The rows the token tensors of M tokens take: a multiple of 16 up to 64 tokens, else of 64.
 int local_rows_padded(int M);
+// Whether a stack over M_pad token rows keeps its norms' sums of squares over each 16 columns, and
+// the floats they take either way.
+constexpr bool local_fine_sums(int M_pad) { return M_pad <= 64; }
+constexpr size_t local_sq_floats(size_t M_pad, size_t hidden) {
+    const size_t fine = 64 * (hidden / 16), spans = M_pad * (hidden / LOCAL_SQ_COLS);
+    return fine > spans ? fine : spans;
+}
 hipError_t launch_local_stack(const LocalArgs& a, const LocalLayer* layers, int nlayers, const float* final_norm,
                               const LocalBuffers& b, hipStream_t stream, DispatchTimer* timer);
 // The dispatches launch_local_stack makes.
-int local_stack_dispatches(const LocalArgs& a, const LocalBuffers& b, int nlayers);
+int local_stack_dispatches(const LocalBuffers& b, int nlayers);
 hipError_t launch_local_embed(const LocalArgs& a, const EmbedArgs& e, int rows, hipStream_t stream, DispatchTimer* timer);
 hipError_t launch_dit_euler(const LocalArgs& a, const EulerArgs& e, int rows, hipStream_t stream, DispatchTimer* timer);
 hipError_t launch_cfm_noise(const float* noise, const float* sampling, float* state, int rows, int len,

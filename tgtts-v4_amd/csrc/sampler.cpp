@@ -183,9 +183,8 @@ tgx_status sampler_create(Context* ctx, const tgx_shape* stack, const tgx_patch_
     A(&smp->x0, Mp * h);
     A(&smp->x, Mp * h);
     A(&smp->h, Mp * h);
-    A(&smp->partial, (size_t)LOCAL_MAX_PARTS * Mp * h);
     A(&smp->normed, Mp * h);
-    A(&smp->row_sq, Mp * (h / LOCAL_SQ_COLS));
+    A(&smp->row_sq, local_sq_floats(Mp, h));
     A(&smp->normed0, Mp * h);
     A(&smp->row_sq0, Mp * (h / LOCAL_SQ_COLS));
     A(&smp->q, Mp * att);
@@ -321,7 +320,7 @@ hipError_t sampler_enqueue(Sampler* s, const float* mu, DispatchTimer* timer, in
     }
     // No `out`: dit_euler takes the final norm of the tokens it reads.
     const LocalBuffers b{s->x0,       s->x,        s->h, s->normed, s->row_sq,   s->normed0, s->row_sq0, s->q, s->k,
-                         s->v,        s->attended, s->mlp, s->partial, nullptr, s->o_parts, s->down_parts};
+                         s->v,        s->attended, s->mlp, nullptr, s->o_parts, s->down_parts};
     const int x_at = COND_AT + F;
     for (size_t i = 0; i < s->step_t.size() && e == hipSuccess; ++i) {
         // in_proj of the patch so far at x_at, and the step's time token (dit.rs:213-219).
@@ -330,8 +329,8 @@ hipError_t sampler_enqueue(Sampler* s, const float* mu, DispatchTimer* timer, in
         e = launch_local_embed(a, step, rows, st, timer);
         ++n;
         if (e == hipSuccess) e = launch_local_stack(a, layers.data(), s->shape.layers, s->final_norm, b, st, timer);
-        n += local_stack_dispatches(a, b, s->shape.layers);
-        EulerArgs eu{s->x, s->row_sq, s->final_norm, s->out_w, s->out_b, s->sampling, s->state, C, F, x_at, s->step_dt[i]};
+        n += local_stack_dispatches(b, s->shape.layers);
+        EulerArgs eu{s->x, s->row_sq, s->final_norm, s->out_w, s->out_b, s->sampling, s->state, C, F, x_at, s->step_dt[i], local_fine_sums(a.M_pad)};
         if (e == hipSuccess) e = launch_dit_euler(a, eu, rows, st, timer);
         ++n;
     }
