@@ -377,6 +377,34 @@ def test_a_fence_spin_changes_how_waits_poll_and_not_what_they_give(ctx):
     o.close()
 
 
+@pytest.mark.parametrize("slack", [1, 1000, 50_000, 123_457])
+def test_a_wait_leaves_the_thread_its_timer_slack(ctx, slack):
+    """Waits sleep with a timer slack of 1 us at most; the thread that waits has its own afterwards,
+    shorter ones untouched."""
+    import ctypes
+    import threading
+
+    from tgx.synth import StackSpec, embeddings
+
+    SET, GET = 29, 30  # PR_SET_TIMERSLACK, PR_GET_TIMERSLACK
+    spec = StackSpec(layers=2, seed=5)
+    x = embeddings(9, "slack", 1, spec.hidden)[0]
+    dec = reference_decoder(ctx, spec, 64, 1)
+    seen = []
+
+    def step():
+        libc = ctypes.CDLL(None)
+        libc.prctl(SET, ctypes.c_ulong(slack), 0, 0, 0)
+        dec.step(0, x)
+        seen.append(libc.prctl(GET, 0, 0, 0, 0))
+
+    t = threading.Thread(target=step)
+    t.start()
+    t.join()
+    dec.close()
+    assert seen == [slack]
+
+
 def test_a_single_dispatch_runs_alone_and_is_timed(ctx):
     """Context::dispatch (context.rs:517-540, as the reference's kernel tests run one kernel): the
     stream-read words as a program gives them, a GPU time, and a refusal with its message."""

@@ -12,8 +12,11 @@
 #include <cmath>
 #include <cstring>
 #include <functional>
+#include <optional>
 #include <thread>
 #include <tuple>
+
+#include <sys/prctl.h>
 
 namespace tgx {
 
@@ -149,16 +152,45 @@ void context_destroy(Context* ctx) {
     delete ctx;
 }
 
+namespace {
+
+// A thread's sleeps end up to its timer slack late, 50 us where nothing set it: many a call's
+// whole work. While a FineSleep lives the calling thread's slack is 1 us; the thread gets its own
+// back. A step's wait ended 35 us late on average with polls 20 us apart and that slack: four
+// steps of one request 2558 us -> 2414 without it, -> 2378 with polls 5 us apart (a four-layer LM
+// 1053 -> 939 -> 890).
+class FineSleep {
+  public:
+    FineSleep() : own_(prctl(PR_GET_TIMERSLACK, 0, 0, 0, 0)) {
+        if (own_ > FINE_NS) prctl(PR_SET_TIMERSLACK, (unsigned long)FINE_NS, 0, 0, 0);
+    }
+    ~FineSleep() {
+        if (own_ > FINE_NS) prctl(PR_SET_TIMERSLACK, (unsigned long)own_, 0, 0, 0);
+    }
+    FineSleep(const FineSleep&) = delete;
+    FineSleep& operator=(const FineSleep&) = delete;
+
+  private:
+    static constexpr int FINE_NS = 1000;
+    const int own_;
+};
+
+}  // namespace
+
 tgx_status wait_event(const Context* ctx, hipEvent_t ev, const char* what) {
     const auto begin = std::chrono::steady_clock::now();
     const auto spin = std::chrono::nanoseconds(ctx ? ctx->fence_spin_ns.load(std::memory_order_relaxed) : 0);
+    std::optional<FineSleep> fine;
     while (true) {
         const hipError_t q = hipEventQuery(ev);
         if (q == hipSuccess) return TGX_OK;
         if (q != hipErrorNotReady) return fail(TGX_E_HIP, std::string(what) + ": " + hipGetErrorString(q));
         const auto waited = std::chrono::steady_clock::now() - begin;
         if (waited > std::chrono::seconds(60)) return fail(TGX_E_TIMEOUT, std::string(what) + " did not finish in 60 s");
-        if (waited >= spin) std::this_thread::sleep_for(std::chrono::microseconds(20));
+        if (waited >= spin) {
+            if (!fine) fine.emplace();
+            std::this_thread::sleep_for(std::chrono::microseconds(5));
+        }
     }
 }
 

@@ -45,7 +45,7 @@ struct Context {
 };
 
 // Waits for `ev`, recorded on the context's stream: polls it without pause for the context's
-// fence spin, then every 20 µs, for 60 s at most (Inner::wait_for, crates/vulkan/src/context.rs:
+// fence spin, then every 5 µs, for 60 s at most (Inner::wait_for, crates/vulkan/src/context.rs:
 // 116-133, and its FENCE_TIMEOUT_NS). TGX_E_HIP for an error the event reports, TGX_E_TIMEOUT
 // past 60 s, each naming `what`.
 tgx_status wait_event(const Context* ctx, hipEvent_t ev, const char* what);
