@@ -393,6 +393,36 @@ def test_a_dit_evaluation_composed_by_kernel_name_is_tgx_sampler_sample_bit_for_
     sampler.close()
 
 
+@pytest.mark.parametrize("rows", [1, 3])
+def test_an_embedding_takes_the_grid_named_for_it_by_256_columns(ctx, rows):
+    """A caller that names local_embed's grid as one workgroup to 256 columns of a row has the bits
+    of one that leaves the grid to the kernel; another grid is refused."""
+    import tgx
+    import tgx.runtime as rt
+
+    rng = np.random.default_rng(rows)
+    h, C, F, T = 1024, FEAT, FRAMES, 1 + FRAMES
+    arrays = [rng.standard_normal(n, dtype=np.float32) for n in (rows * C * F, h * C, h, h)]
+    mem = [rt.Memory(ctx, a.nbytes) for a in arrays]
+    for m, a in zip(mem, arrays):
+        m.write(a)
+    pad = (rows * T + 15) // 16 * 16
+    c = [rows * T, T, h, 4096, 16, 2, rt.f32_bits(1e-5), 1] + [rows, C, F, 1, 0, 1, 0, 1, 1]
+    got = []
+    for groups in ((0, 0, 0), (h // 256, rows, 1)):
+        x0 = rt.Memory(ctx, pad * h * 4)
+        rt.dispatch(ctx, "local_embed", [*mem, None, x0, None, None], c, groups)
+        got.append(x0.read(np.uint32, rows * T * h))
+        x0.close()
+    assert np.array_equal(*got) and got[0].any()
+    x0 = rt.Memory(ctx, pad * h * 4)
+    with pytest.raises(tgx.TgxError):
+        rt.dispatch(ctx, "local_embed", [*mem, None, x0, None, None], c, (h // 128, rows, 1))
+    x0.close()
+    for m in mem:
+        m.close()
+
+
 def test_the_wider_kernels_refuse_on_the_host_what_they_could_not_run(ctx):
     """Each kernel past the decode step checks its constants and every binding's bytes before
     anything is recorded (Kernels::check, crates/graph/src/kernels.rs), as the decode kernels do."""

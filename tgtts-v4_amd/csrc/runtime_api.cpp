@@ -57,6 +57,7 @@ struct Bound {
 struct Launch {
     const char* name = nullptr;
     KernelLaunch k;
+    dim3 also{0, 0, 0};  // a grid the kernel's work was once cut by, taken for k.grid when a caller names it
     DecodeArgs a{};
     LayerArgs l{};
     ResidualArgs r{};
@@ -853,6 +854,7 @@ tgx_status build_local_embed(const Bound* b, const uint32_t* c, Launch* L) {
     e.gain = (const float*)b[4].ptr;
     e.normed = (uint16_t*)b[6].ptr;
     e.row_sq = (float*)b[7].ptr;
+    L->also = dim3(a.hidden / 256, rows);
     return capture_one("local_embed", [&] { return launch_local_embed(a, e, (int)rows, nullptr, nullptr); }, L);
 }
 
@@ -1452,7 +1454,8 @@ tgx_status tgx_program_launch(tgx_program* prog, const tgx_dispatch* d) {
     TGX_TRY(k->build(bound.data(), d->constants, L.get()));
     if (!L->k.func) return fail(TGX_E_KERNELS, who + "no instance for these constants");
     const bool derive = d->groups[0] == 0 && d->groups[1] == 0 && d->groups[2] == 0;
-    if (!derive && (d->groups[0] != L->k.grid.x || d->groups[1] != L->k.grid.y || d->groups[2] != L->k.grid.z))
+    auto names = [&](const dim3& g) { return d->groups[0] == g.x && d->groups[1] == g.y && d->groups[2] == g.z; };
+    if (!derive && !names(L->k.grid) && !names(L->also))
         return fail(TGX_E_SHAPE, who + "a grid of " + std::to_string(d->groups[0]) + " x " + std::to_string(d->groups[1]) + " x " +
                                      std::to_string(d->groups[2]) + " where the kernel takes " + std::to_string(L->k.grid.x) + " x " +
                                      std::to_string(L->k.grid.y) + " x " + std::to_string(L->k.grid.z));
