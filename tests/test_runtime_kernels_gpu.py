@@ -423,6 +423,46 @@ def test_an_embedding_takes_the_grid_named_for_it_by_256_columns(ctx, rows):
         m.close()
 
 
+@pytest.mark.parametrize("rows", [1, 5, 16, 17])
+@pytest.mark.parametrize("K, N", [(1024, 1024), (2048, 1056), (4096, 2048), (6144, 2048)])
+def test_residual_strips_of_4_and_16_rows_give_the_same_bits(ctx, K, N, rows):
+    """gemv_residual over 4-row strips, one to a workgroup up to 256 of them (N 1024) and two past
+    (N 1056, 2048), and over 16-row strips: the same bits, the 16-column sums of squares the 4-column
+    ones added in order; `out` within f32 sums of K products of the exact product (K 2^-24 of the
+    sum of magnitudes), by the kernel's grid or one workgroup a strip, as a caller may name it."""
+    import tgx.runtime as rt
+
+    rng = np.random.default_rng(K + N + rows)
+    bf16 = lambda a: (a.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    w, x = bf16(rng.standard_normal((N, K)) / 32), bf16(rng.standard_normal((rows, K)))
+    residual, gain = rng.standard_normal((rows, N), dtype=np.float32), rng.standard_normal(N, dtype=np.float32)
+    xm, rm, gm = rt.Memory(ctx, x.nbytes), rt.Memory(ctx, residual.nbytes), rt.Memory(ctx, gain.nbytes)
+    xm.write(np.ascontiguousarray(x.reshape(rows, K // 32, 32).transpose(1, 0, 2)))
+    rm.write(residual)
+    gm.write(gain)
+    got = {}
+    for strip, tiles, named in ((4, rt.TILES_4, False), (4, rt.TILES_4, True), (16, rt.TILES_16, False)):
+        wm = rt.Memory(ctx, w.nbytes)
+        wm.write_tiles(w, tiles)
+        out, out_n, sq = rt.Memory(ctx, rows * N * 4), rt.Memory(ctx, rows * N * 2), rt.Memory(ctx, rows * (N // strip) * 4)
+        c = [1024, 4096, 16, 2, rows, 64, rows, 1, rows, rt.f32_bits(1e-5), 1, 64, K, N, strip]
+        rt.dispatch(ctx, "gemv_residual", [xm, wm, rm, gm, out, out_n, sq], c, (N // strip, (rows + 15) // 16, 1) if named else (0, 0, 0))
+        got[strip, named] = [out.read(np.float32, rows * N), out_n.read(np.uint32, rows * N // 2),
+                             sq.read(np.float32, rows * (N // strip)).reshape(rows, -1)]
+        for m in (wm, out, out_n, sq):
+            m.close()
+    for m in (xm, rm, gm):
+        m.close()
+    (out, out_n, sq), named, (out16, out_n16, sq16) = got[4, False], got[4, True], got[16, False]
+    assert all(np.array_equal(a, b) for a, b in zip(got[4, False], named))
+    assert np.array_equal(out, out16) and np.array_equal(out_n, out_n16)
+    s = sq.reshape(rows, -1, 4)
+    assert np.array_equal(((s[..., 0] + s[..., 1]) + s[..., 2]) + s[..., 3], sq16)
+    w64, x64 = bf16_to_f32(w).astype(np.float64), bf16_to_f32(x).astype(np.float64)
+    bound = K * 2.0**-24 * (np.abs(x64) @ np.abs(w64).T + np.abs(residual))
+    assert (np.abs(out.reshape(rows, N) - (residual + x64 @ w64.T)) <= bound).all()
+
+
 def test_the_wider_kernels_refuse_on_the_host_what_they_could_not_run(ctx):
     """Each kernel past the decode step checks its constants and every binding's bytes before
     anything is recorded (Kernels::check, crates/graph/src/kernels.rs), as the decode kernels do."""

@@ -183,9 +183,9 @@ struct RowSquares {
     }
 };
 
-// One wave's chains for strips `strip[s]` (R rows each, in MFMA rows 0..R-1) of W [N][CH chunks]
-// against its k-blocks of the tile, k-block after k-block.
-template <int S, int CH, int R = 16>
+// One wave's chains for strips `strip[s]` (R rows each, in MFMA rows 0..R-1; with G, G strips one after
+// another from strip[s]) of W [N][CH chunks] against its k-blocks of the tile, k-block after k-block.
+template <int S, int CH, int R = 16, int G = 1>
 struct Gemv {
     static constexpr int KB = CH * PER_WAVE;
     f32x4 acc[S];
@@ -194,8 +194,9 @@ struct Gemv {
     __device__ void load(const uint16_t* __restrict__ w, const int (&strip)[S]) {
         constexpr int kblocks = CH * CHUNK_KB;
         const int lane = threadIdx.x % WAVE;
-        // Lanes past the strip's rows read its last row again.
-        const int off = weight_lane_offset((lane / 16) * 16 + min(lane % 16, R - 1), R);
+        // Lanes past the strips' rows read the last row again.
+        const int row = min(lane % 16, R * G - 1);
+        const int off = (int)weight_tile_index(row / R, 0, kblocks, R) + weight_lane_offset((lane / 16) * 16 + row % R, R);
 #pragma unroll
         for (int i = 0; i < KB; ++i)
 #pragma unroll
@@ -407,32 +408,32 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_gate_up(DecodeArgs a, Layer
 }
 
 // ---------------------------------------------------------------------------------------------
-// gemv_residual: out = residual + W x, workgroup (strip, tile): a strip of R rows over the whole
-// of K. The epilogue's thread (c, q) (tile row c, rows 4 q .. 4 q + 3 of the strip; the first
-// 4 R threads) loads its residual and next-norm gains first of all, and with next_norm set also
-// writes out next_norm in bf16 and the sum of squares of the strip's R columns of row c: its 4 in
+// gemv_residual: out = residual + W x, workgroup (strips, tile): G strips of R rows over the whole
+// of K. The epilogue's thread (c, q) (tile row c, rows 4 q .. 4 q + 3 of the strips; the first
+// 4 R G threads) loads its residual and next-norm gains first of all, and with next_norm set also
+// writes out next_norm in bf16 and the sum of squares of each strip's R columns of row c: its 4 in
 // order, and at R = 16 the four threads' sums added in column order (the order a 4-column reader
 // adds them in).
-template <int CH, int R>
+template <int CH, int R, int G>
 __global__ void __launch_bounds__(GEMV_THREADS) gemv_residual(DecodeArgs a, ResidualArgs r) {
-    constexpr int EPI = 16 * (R / SQ_COLS);
+    constexpr int ROWS = R * G;
+    constexpr int EPI = 16 * (ROWS / SQ_COLS);
     constexpr int LOADERS = EPI < WAVE ? WAVE : EPI;  // whole waves load (past EPI, the same again)
     static_assert(LOADERS % WAVE == 0, "whole waves");
     __shared__ f32x4 red[GEMV_WAVES * 64];
-    const int strip_id = blockIdx.x, tile = blockIdx.y;
-    const int strip[1] = {strip_id};
-    const int c = threadIdx.x % 16, q = (threadIdx.x / 16) % (R / SQ_COLS);
+    const int tile = blockIdx.y;
+    const int c = threadIdx.x % 16, q = (threadIdx.x / 16) % (ROWS / SQ_COLS);
     const int b = tile * 16 + c;
-    const int n0 = strip_id * R + q * SQ_COLS;
+    const int n0 = blockIdx.x * ROWS + q * SQ_COLS;
     float4 res = make_float4(0.f, 0.f, 0.f, 0.f), gain = res;
     if (threadIdx.x < LOADERS) {
         res = load_f4(r.residual + (size_t)min(b, a.rows - 1) * r.N + n0);
         gain = load_f4((r.next_norm ? r.next_norm : r.residual) + n0);
     }
     RawRows<CH> x;
-    Gemv<1, CH, R> g;
+    Gemv<1, CH, R, G> g;
     x.load(r.x, a.rows, tile);
-    g.load(r.w, strip);
+    g.load(r.w, {(int)blockIdx.x * G});
     all_issued();
     g.run(x.xf);
     spill<1>(g.acc, red);
@@ -458,7 +459,7 @@ __global__ void __launch_bounds__(GEMV_THREADS) gemv_residual(DecodeArgs a, Resi
     if (r.next_norm) {
         *reinterpret_cast<uint2*>(r.out_n + operand_index(b, n0, a.rows)) =
             make_uint2(pack_bf16x2(v.x * gain.x, v.y * gain.y), pack_bf16x2(v.z * gain.z, v.w * gain.w));
-        if (q == 0) r.out_sq[(size_t)b * (r.N / R) + strip_id] = s2;
+        if (q * SQ_COLS % R == 0) r.out_sq[(size_t)b * (r.N / R) + n0 / R] = s2;
     }
 }
 
@@ -810,8 +811,9 @@ struct Qkv {
 };
 template <int CH> struct PickGateUp { static auto get() { return gemv_gate_up<hidden_ch(CH), 1>; } };
 template <int CH> struct PickGateUpWide { static auto get() { return gemv_gate_up<hidden_ch(CH), 1, true>; } };
-template <int CH> struct PickResidual4 { static auto get() { return gemv_residual<CH, 4>; } };
-template <int CH> struct PickResidual16 { static auto get() { return gemv_residual<CH, 16>; } };
+template <int CH> struct PickResidual4 { static auto get() { return gemv_residual<CH, 4, 1>; } };
+template <int CH> struct PickResidual4x2 { static auto get() { return gemv_residual<CH, 4, 2>; } };
+template <int CH> struct PickResidual16 { static auto get() { return gemv_residual<CH, 16, 1>; } };
 template <int CH> struct PickFinal { static auto get() { return final_rmsnorm<hidden_ch(CH)>; } };
 
 // The kernel of `launch` with its arguments `params`, timed by the timer's next events when given.
@@ -855,16 +857,21 @@ size_t decode_chain_floats(const DecodeArgs& a) {
     return (size_t)a.rows * a.kv_heads * ATTN_WAVES * chain_floats(a.heads / a.kv_heads, a.head_dim);
 }
 
+// Past a 4-row strip for every CU a workgroup takes two: a wave's loads of K 6144 fill the registers of
+// a CU with one workgroup, so that twice the CUs' workgroups run one after another, and the two strips
+// share an MFMA's rows and the reads of x. us at hidden 2048 and 8 rows: down_proj (K 6144) 10.9 -> 7.2
+// (2.3 -> 3.5 TB/s), o_proj (K 2048) 4.9 -> 4.2; one row 10.1 -> 6.8 and 4.9 -> 4.4.
+constexpr int RESIDUAL_STRIPS_MOST = 256;
+
 KernelLaunch residual_launch(const DecodeArgs& a, const ResidualArgs& r) {
     const int chunks = r.K / CHUNK_COLS;
     KernelLaunch k;
-    if (r.R == 4)
-        k.func = (const void*)by_chunks<PickResidual4>(chunks);
-    else if (r.R == 16)
-        k.func = (const void*)by_chunks<PickResidual16>(chunks);
-    else
-        return k;
-    k.grid = dim3(r.N / r.R, decode_tiles(a.rows));
+    if (r.R != 4 && r.R != 16) return k;
+    const int strips = r.R == 4 && r.N / 4 > RESIDUAL_STRIPS_MOST ? 2 : 1;  // to a workgroup
+    k.func = strips == 2 ? (const void*)by_chunks<PickResidual4x2>(chunks)
+             : r.R == 4  ? (const void*)by_chunks<PickResidual4>(chunks)
+                         : (const void*)by_chunks<PickResidual16>(chunks);
+    k.grid = dim3(r.N / (r.R * strips), decode_tiles(a.rows));
     k.block = dim3(GEMV_THREADS);
     return k;
 }

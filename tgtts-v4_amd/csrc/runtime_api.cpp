@@ -286,6 +286,7 @@ tgx_status build_residual(const Bound* b, const uint32_t* c, Launch* L) {
     L->a = a;
     L->r = r;
     L->k = residual_launch(a, r);
+    L->also = dim3(N / Rs, decode_tiles(a.rows));
     L->params[0] = &L->a;
     L->params[1] = &L->r;
     return TGX_OK;
