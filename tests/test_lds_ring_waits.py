@@ -250,6 +250,24 @@ def test_local_ring_reads_no_slot_before_it_lands():
         check(runs, f"local_gemm_ring<{LOCAL_EPI[epi]}, {sw}, {kbp}, {parts}, {tt}> K {K} N {N}")
 
 
+def test_local_parts_read_no_slot_before_it_lands():
+    kernels = assembly("local_kernels.hip")
+    symbols = instances(kernels, "local_gemm_parts")
+    assert symbols
+    L = layout("local_kernels.hip")
+    for symbol in symbols:
+        (kbp, parts), tt = template_args(symbol), 2
+        M, M_pad, K, N = 345, 384, kbp * parts * 32, 1024
+        a = lr.pack(L, "LocalArgs", dict(M=M, M_pad=M_pad, T=5, hidden=1024, inner=4096, heads=16, kv_heads=2, eps=f32(1e-5),
+                                         scale=f32(0.125), rope=1, cos=COS, sin=SIN))
+        g = dict(w=W, x=X, K=K, N=N, partial=0, mlp=0, q=0, k=0, v=0, row_sq=0, residual=AUX, sum=OUT, next_gain=AUX + 0x100000,
+                 normed=OUT + 0x1000000, sum_sq=OUT + 0x2000000)
+        grid = (N // 64, M_pad // (16 * tt), 1)
+        last = (grid[0] - 1, (M - 1) // (16 * tt), 0)
+        runs = replay(kernels[symbol], [a, lr.pack(L, "LocalGemm", g)], grid, 128 * parts, {}, [(0, 0, 0), last])
+        check(runs, f"local_gemm_parts<{kbp}, {parts}> K {K}")
+
+
 def test_the_local_rings_prelude_without_its_scheduling_barriers_is_caught(tmp_path):
     """Planted defect: the prelude as it was before its scheduling barriers (every group's loads
     issued in one stretch, which the compiler reorders), which let the first waits pass a slot's

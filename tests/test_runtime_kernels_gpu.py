@@ -423,6 +423,43 @@ def test_an_embedding_takes_the_grid_named_for_it_by_256_columns(ctx, rows):
         m.close()
 
 
+@pytest.mark.parametrize("K, parts", [(1024, 2), (2048, 2), (2048, 4), (4096, 4)])
+def test_parts_added_over_few_tokens_have_the_bits_of_those_over_many(ctx, K, parts):
+    """local_gemm_add_norm up to 512 tokens (a part to a pair of waves) and past them (every part in
+    each wave): a token's sums, next norm's input and sums of squares are the same bits, with the
+    last tile full, part full (70, 507 tokens) and alone (65)."""
+    import tgx.runtime as rt
+
+    rng = np.random.default_rng(K + parts)
+    bf16 = lambda a: (a.astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+    h, most = 1024, 576
+    w, x = bf16(rng.standard_normal((h, K)) / 32), bf16(rng.standard_normal(most * K))  # in fragment order
+    residual, gain = rng.standard_normal(most * h, dtype=np.float32), rng.standard_normal(h, dtype=np.float32)
+    wm, gm = rt.Memory(ctx, w.nbytes), rt.Memory(ctx, gain.nbytes)
+    wm.write_tiles(w, rt.TILES_16)
+    gm.write(gain)
+    want = None
+    for tokens in (most, 65, 70, 507, 512):
+        pad = (tokens + 63) // 64 * 64
+        xm, rm = rt.Memory(ctx, pad * K * 2), rt.Memory(ctx, pad * h * 4)
+        xm.write(x[:pad * K])
+        rm.write(residual[:pad * h])
+        out, normed, sq = rt.Memory(ctx, pad * h * 4), rt.Memory(ctx, pad * h * 2), rt.Memory(ctx, pad * 16 * 4)
+        c = [tokens, 1, h, 4096, 16, 2, rt.f32_bits(1e-5), 1, K, h, parts]
+        # The grid left to the kernel, or named as a workgroup to 64 tokens.
+        groups = (h // 64, pad // 64, 1) if tokens == 507 else (0, 0, 0)
+        rt.dispatch(ctx, "local_gemm_add_norm", [xm, wm, rm, gm, out, normed, sq], c, groups)
+        full = tokens // 16 * 16  # fragments are of 16 tokens
+        got = [out.read(np.uint32, tokens * h), normed.read(np.uint32, full * h // 2), sq.read(np.uint32, tokens * 16)]
+        for m in (xm, rm, out, normed, sq):
+            m.close()
+        want = got if want is None else want
+        for g, all_of_them in zip(got, want):
+            assert np.array_equal(g, all_of_them[:len(g)]), tokens
+    wm.close()
+    gm.close()
+
+
 @pytest.mark.parametrize("rows", [1, 5, 16, 17])
 @pytest.mark.parametrize("K, N", [(1024, 1024), (2048, 1056), (4096, 2048), (6144, 2048)])
 def test_residual_strips_of_4_and_16_rows_give_the_same_bits(ctx, K, N, rows):

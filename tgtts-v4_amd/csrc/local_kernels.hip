@@ -4,14 +4,15 @@
 //
 //   local_gemm      C = X W^T over up to a few hundred tokens, bf16 in, f32 accumulate: up to 64
 //                   tokens straight from memory into each wave's registers beside its strips of
-//                   W (local_gemm_direct); more in 64-token tiles streamed through a ring of LDS
-//                   slots, read by the waves of a workgroup that each stream their own strips of
-//                   W (local_gemm_ring). The epilogue fused: the row's RMSNorm scale with RoPE at
-//                   each token's place in its sequence (local_qkv_rope.comp), the same scale with
-//                   SiLU(gate) up (local_gate_up.comp), the f32 sums of one part of the columns
-//                   (local_partial.comp), or over more than 64 tokens the parts added, the
-//                   residual added and the next norm's input with its sums of squares
-//                   (local_add_norm.comp)
+//                   W (local_gemm_direct; with o_proj's and down_proj's parts added,
+//                   local_gemm_sum); more in tiles streamed through a ring of LDS slots, read by
+//                   the waves of a workgroup that each stream their own strips of W
+//                   (local_gemm_ring; a part of K to a pair of waves, local_gemm_parts). The
+//                   epilogue fused: the row's RMSNorm scale with RoPE at each token's place in
+//                   its sequence (local_qkv_rope.comp), the same scale with SiLU(gate) up
+//                   (local_gate_up.comp), the f32 sums of one part of the columns
+//                   (local_partial.comp), or the parts added, the residual added and the next
+//                   norm's input with its sums of squares (local_add_norm.comp)
 //   local_attention every token of a sequence attends to every token of it, a wave to a
 //                   sequence and query head, both products on MFMA (local_attention.comp)
 //   local_add_norm  residual + the parts' sums in their order, then the next norm's input
@@ -532,6 +533,126 @@ __global__ void __launch_bounds__(4 * WAVE) __attribute__((amdgpu_waves_per_eu(2
     }
 }
 
+// local_gemm_parts, o_proj and down_proj for more than 64 tokens while the chip takes every workgroup at
+// once: 2 P waves to 32 tokens and 64 columns, a pair of waves to each of the P parts of K, wave h of a
+// pair to two of the four strips against both token tiles. A pair's k-blocks go through a ring of LDS
+// slots of its own as local_gemm_ring's go through its one, and the pairs run side by side: each chain is
+// a part's k-blocks long, and a fragment of a token tile in LDS feeds two strips. At the end the parts'
+// sums meet in LDS and the waves take a strip's tile each, the parts added in part order, then
+// local_gemm_ring's epilogue, its residual fetched before the ring: the same bits. What bounds it is the
+// 6 KiB a k-block that a workgroup's loads bring one CU (145 GB/s). us at 66 / 352 / 506 tokens: down_proj
+// (K 4096) 12.2 / 12.5 / 13.2 by the ring -> 9.9 / 10.9 / 11.3, o_proj (K 1024) 5.7 / 6.2 / 7.8 -> 4.9 /
+// 5.8 / 6.6; four token tiles a workgroup 13.3 / 13.5 / 13.4 and 6.8 / 7.8 / 7.7.
+// Grid (N / 64, M_pad / 32).
+constexpr int PARTS_TT = 2;
+constexpr int parts_depth(int parts) { return 128 / (parts * PARTS_TT) < 12 ? 128 / (parts * PARTS_TT) : 12; }
+constexpr size_t parts_lds(int parts) {
+    return (size_t)parts_depth(parts) * parts * PARTS_TT * 64 * sizeof(uint4) + 4 * 16 * PARTS_TT * sizeof(float);
+}
+template <int KBP, int P>
+__global__ void __launch_bounds__(2 * P * WAVE) local_gemm_parts(LocalArgs a, LocalGemm g) {
+    constexpr int SW = 2, TT = PARTS_TT, RING = parts_depth(P);
+    constexpr int XL = TT / 2;      // token tiles a wave loads
+    constexpr int GROUP = SW + XL;  // a wave's loads of a k-block
+    constexpr int ITEMS = 4 * TT / (2 * P);  // blocks of a strip and a tile to a wave at the end
+    static_assert(TT % 2 == 0 && 4 * TT % (2 * P) == 0 && (2 * P) % 4 == 0, "the tiles of a pair, a strip to a wave at the end");
+    static_assert(KBP >= RING && RING * GROUP + ITEMS + 1 < 64, "the loads in flight fit the wave's count");
+    static_assert((size_t)P * 4 * TT * 64 * sizeof(f32x4) <= (size_t)RING * P * TT * 64 * sizeof(uint4), "the sums fit the ring");
+    extern __shared__ uint4 xs[];  // [P][RING][TT tiles][64 lanes], then the parts' sums
+    float* sq_part = reinterpret_cast<float*>(xs + RING * P * TT * 64);  // [4 strips][16 TT tokens]
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE, quad = lane / 16;
+    const int part = wv / 2, h = wv % 2;
+    const int m0 = blockIdx.y * 16 * TT;
+    if (m0 >= a.M) return;  // padding alone
+    // What the epilogue reads, ahead of the groups.
+    const int es = wv % 4, n = (blockIdx.x * 4 + es) * 16 + quad * 4;  // its strip's columns
+    float4 gn = make_float4(0.f, 0.f, 0.f, 0.f), res[ITEMS];
+    gn = *reinterpret_cast<const float4*>((g.next_gain ? g.next_gain : g.residual) + n);
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i)
+        res[i] = *reinterpret_cast<const float4*>(g.residual + (size_t)(m0 + 16 * (wv / 4 + i * (P / 2)) + lane % 16) * g.N + n);
+    const int strip[SW] = {(int)blockIdx.x * 4 + 2 * h, (int)blockIdx.x * 4 + 2 * h + 1};
+    WeightRing<SW, KBP, RING> w;
+    w.start(g, strip, part * KBP, lane);
+    // Tiles h, h + 2 ..'s fragments, 1 KiB each.
+    const uint16_t* xp = g.x + act_index(m0 + 16 * h, part * KBP * 32, g.K) + lane * 8;
+    const size_t tile2 = (size_t)2 * (g.K / 32) * 512;  // two tiles on
+    uint4* slots = xs + part * RING * TT * 64;
+    auto fetch = [&](int kb) __attribute__((always_inline)) {
+        w.fetch(kb, kb + 1);
+#pragma unroll
+        for (int j = 0; j < XL; ++j) load_to_lds(xp + j * tile2 + kb * 512, &slots[((kb % RING) * TT + h + 2 * j) * 64]);
+    };
+    // Each group behind the loads before it, as in local_gemm_ring.
+    all_issued();
+#pragma unroll
+    for (int kb = 0; kb < RING; ++kb) {
+        fetch(kb);
+        all_issued();
+    }
+    f32x4 acc[SW][TT];
+#pragma unroll
+    for (int s = 0; s < SW; ++s)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[s][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    wait_vm_seen<(RING - 1) * GROUP>();
+    stage_barrier();
+    uint4 xf[2][TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xf[0][t] = lds_read16(&slots[t * 64 + lane]);
+#pragma unroll
+    for (int kb = 0; kb < KBP; ++kb) {
+        const int b = kb % 2;
+        lds_landed(xf[b]);
+        if (kb + 1 < KBP) {
+            wait_vm_at_most<(RING - 2) * GROUP>(GROUP * (RING - 2 < KBP - 2 - kb ? RING - 2 : KBP - 2 - kb));
+            stage_barrier();
+#pragma unroll
+            for (int t = 0; t < TT; ++t) xf[1 - b][t] = lds_read16(&slots[(((kb + 1) % RING) * TT + t) * 64 + lane]);
+        }
+#pragma unroll
+        for (int s = 0; s < SW; ++s)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) acc[s][t] = mfma16(w.wf[kb % RING][s], xf[b][t], acc[s][t]);
+        if (kb + RING < KBP) fetch(kb + RING);
+        all_issued();
+    }
+    // Every wave has read its last slot; the parts' sums, [part][tile][strip][lane].
+    stage_barrier();
+    f32x4* sums = reinterpret_cast<f32x4*>(xs);
+#pragma unroll
+    for (int s = 0; s < SW; ++s)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) sums[((part * TT + t) * 4 + 2 * h + s) * 64 + lane] = acc[s][t];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        const int t = wv / 4 + i * (P / 2), m = m0 + 16 * t + lane % 16;
+        f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int p = 0; p < P; ++p) sum += sums[((p * TT + t) * 4 + es) * 64 + lane];
+        const float4 v = make_float4(res[i].x + sum[0], res[i].y + sum[1], res[i].z + sum[2], res[i].w + sum[3]);
+        if (m < a.M) {
+            *reinterpret_cast<float4*>(g.sum + (size_t)m * g.N + n) = v;
+            if (g.next_gain)
+                *reinterpret_cast<uint2*>(g.normed + act_index(m, n, g.N)) =
+                    make_uint2(pack_bf16x2(v.x * gn.x, v.y * gn.y), pack_bf16x2(v.z * gn.z, v.w * gn.w));
+        }
+        float s4 = squares4(v.x, v.y, v.z, v.w);
+        s4 += lane_xor16(s4);
+        s4 += lane_xor32(s4);
+        if (quad == 0) sq_part[es * 16 * TT + 16 * t + lane] = s4;
+    }
+    if (!g.next_gain) return;
+    __syncthreads();
+    if (threadIdx.x < 16 * TT) {
+        const int m = m0 + threadIdx.x;
+        const float* q = sq_part + threadIdx.x;
+        const float s = (q[0] + q[16 * TT]) + (q[2 * 16 * TT] + q[3 * 16 * TT]);
+        if (m < a.M) g.sum_sq[(size_t)m * SQ_PARTS + blockIdx.x] = s;
+    }
+}
+
 // The GEMM of a projection whose epilogue is one of QKV, SILU or PARTIAL: `units` work units of
 // SW strips (gate/up: pairs of strips), each output summed over the KBP k-blocks of its part. At
 // most 64 tokens take the direct GEMM, more the ring (QKV and SILU only: its parts are added in
@@ -582,10 +703,28 @@ void local_sum(const char* label, const LocalArgs& a, const LocalGemm& g, int kb
         dispatch(label, local_gemm_sum<32, 4>, grid, block, 0, stream, timer, a, g);
 }
 
-// o_proj and down_proj over more than 64 tokens: the ring with the parts added and the residual
+constexpr int PARTS_WORKGROUPS = 256;
+
+// o_proj and down_proj over more than 64 tokens: local_gemm_parts, or the ring with the parts added and the residual
 // added in its epilogue (LEPI_ADD), 16 or 32 k-blocks to each of 2 or 4 parts.
 void local_gemm_add(const char* label, const LocalArgs& a, const LocalGemm& g, int kbp, int parts, hipStream_t stream,
                     DispatchTimer* timer) {
+    // local_gemm_parts while each workgroup has a CU; past that its smaller tiles' reads cost more (528
+    // tokens: down_proj 18.7 us against the ring's 12.9).
+    const int columns = g.N / 64;
+    if (columns * ((a.M + 16 * PARTS_TT - 1) / (16 * PARTS_TT)) <= PARTS_WORKGROUPS) {
+        const dim3 grid(columns, a.M_pad / (16 * PARTS_TT)), block(2 * parts * WAVE);
+        const size_t lds = parts_lds(parts);
+        if (kbp == 16 && parts == 2)
+            dispatch(label, local_gemm_parts<16, 2>, grid, block, lds, stream, timer, a, g);
+        else if (kbp == 32 && parts == 2)
+            dispatch(label, local_gemm_parts<32, 2>, grid, block, lds, stream, timer, a, g);
+        else if (kbp == 16 && parts == 4)
+            dispatch(label, local_gemm_parts<16, 4>, grid, block, lds, stream, timer, a, g);
+        else
+            dispatch(label, local_gemm_parts<32, 4>, grid, block, lds, stream, timer, a, g);
+        return;
+    }
     const dim3 grid(g.N / 64, a.M_pad / 64), block(4 * WAVE);
     const size_t lds = ring_lds(1, 4);
     if (kbp == 16 && parts == 2)
@@ -602,6 +741,11 @@ template <int EPI, int SW, int KBP, int P, int TT = 4>
 hipError_t local_ring_lds() {
     return hipFuncSetAttribute((const void*)local_gemm_ring<EPI, SW, KBP, P, TT>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)ring_lds(SW, TT));
+}
+
+template <int KBP, int P>
+hipError_t local_parts_lds() {
+    return hipFuncSetAttribute((const void*)local_gemm_parts<KBP, P>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)parts_lds(P));
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1087,6 +1231,10 @@ hipError_t local_prepare() {
     if (e == hipSuccess) e = local_ring_lds<LEPI_ADD, 1, 32, 2>();
     if (e == hipSuccess) e = local_ring_lds<LEPI_ADD, 1, 16, 4>();
     if (e == hipSuccess) e = local_ring_lds<LEPI_ADD, 1, 32, 4>();
+    if (e == hipSuccess) e = local_parts_lds<16, 2>();
+    if (e == hipSuccess) e = local_parts_lds<32, 2>();
+    if (e == hipSuccess) e = local_parts_lds<16, 4>();
+    if (e == hipSuccess) e = local_parts_lds<32, 4>();
     return e;
 }
 

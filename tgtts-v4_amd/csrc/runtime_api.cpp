@@ -780,6 +780,7 @@ tgx_status build_local_gemm_add_norm(const Bound* b, const uint32_t* c, Launch* 
     g.sum = (float*)b[4].ptr;
     g.normed = (uint16_t*)b[5].ptr;
     g.sum_sq = (float*)b[6].ptr;
+    L->also = dim3(N / 64, a.M_pad / 64);
     return capture_one("local_gemm_add_norm", [&] { return launch_local_add(a, g, (int)parts, nullptr, nullptr); }, L);
 }
 
