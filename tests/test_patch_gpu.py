@@ -501,6 +501,24 @@ def test_an_encoder_of_any_rows_matches_the_oracle_and_gives_the_same_bits(ctx, 
         np.testing.assert_array_equal(got, most[:n])
 
 
+@pytest.mark.parametrize("rows", [11, 12, 18, 23, 24])
+def test_a_sampler_of_many_rows_gives_a_request_its_bits_alone(ctx, rows):
+    """242, 264, 396, 506 and 528 tokens: gate/up by four token tiles a workgroup and by eight (the last
+    eight half empty at 264 and 396), o_proj and down_proj by parts and by the ring."""
+    from tgx.synth import sampler_weights
+
+    spec = _dit_spec(layers=2)
+    w = sampler_weights(spec, FEAT)
+    mu, cond, noise, sampling = _inputs(rows)
+    s = _sampler(ctx, rows, spec, w)
+    got = s.sample(mu, cond, noise, sampling)
+    s.close()
+    one = _sampler(ctx, 1, spec, w)
+    for r in (0, 1, rows - 2, rows - 1):
+        np.testing.assert_array_equal(one.sample(mu[r:r + 1], cond[r:r + 1], noise[r:r + 1], sampling[r:r + 1])[0], got[r])
+    one.close()
+
+
 def test_samplers_around_64_tokens_give_a_request_the_same_bits(ctx):
     """Two requests' 44 tokens go through the kernels for at most 64, three's 66 through the ring's."""
     from tgx.synth import sampler_weights

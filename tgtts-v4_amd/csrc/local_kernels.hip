@@ -416,12 +416,14 @@ __global__ void __launch_bounds__(4 * WAVE) __attribute__((amdgpu_waves_per_eu(2
     // each wave's count of loads is the same) go out before the groups: the wait for the first
     // group covers them.
     RowSq sq;
-    if (SCALED) sq.load(g.row_sq, m0 + 64 * (wv % XL) + lane);
+    // Eight tiles' second four may lie past the padded tokens: the first four again, never stored.
+    const bool whole = TT == 4 || m0 + 64 < a.M_pad;
+    if (SCALED) sq.load(g.row_sq, m0 + (whole ? 64 * (wv % XL) : 0) + lane);
     WeightRing<SW, KB, RING> w;
     w.start(g, strip, 0, lane);
     // Tiles wv, wv + 4 ..'s fragments, 1 KiB each.
     const uint16_t* xp = g.x + act_index(m0 + 16 * wv, 0, g.K) + lane * 8;
-    const size_t tile4 = (size_t)4 * (g.K / 32) * 512;  // four tiles on
+    const size_t tile4 = whole ? (size_t)4 * (g.K / 32) * 512 : 0;  // four tiles on
     auto fetch = [&](int kb) __attribute__((always_inline)) {
         w.fetch(kb, kb + 1);
 #pragma unroll
@@ -676,11 +678,12 @@ void local_gemm(const char* label, const LocalArgs& a, const LocalGemm& g, int u
         }
         return direct(std::false_type{});
     }
-    // Eight token tiles a workgroup for gate/up where the tokens come in 128s (its W, 16 MiB at
-    // the sampler's shape, is the most read); four otherwise.
+    // Four token tiles a workgroup while each has a CU, eight past that for gate/up (its W, 16 MiB at
+    // the sampler's shape, is the most read). us at 198 / 242 tokens 8.1 / 8.0 by four and 10.3 / 10.1 by
+    // eight; 264 / 396 / 528 / 1408 tokens 11.3 / 11.7 / 15.6 / 29.0 and 9.5 / 9.5 / 13.7 / 22.8.
     if constexpr (EPI == LEPI_SILU) {
-        if (a.M_pad % 128 == 0) {
-            dispatch(label, local_gemm_ring<EPI, SW, KBP, 1, 8>, dim3(units / 4, a.M_pad / 128), dim3(4 * WAVE), ring_lds(SW, 8),
+        if (units / 4 * (a.M_pad / 64) > 256) {
+            dispatch(label, local_gemm_ring<EPI, SW, KBP, 1, 8>, dim3(units / 4, (a.M_pad + 127) / 128), dim3(4 * WAVE), ring_lds(SW, 8),
                      stream, timer, a, g);
             return;
         }
