@@ -676,6 +676,12 @@ class Replay:
             res, scc = t & M32, t < 0
         elif op == "mul_i32":
             res = (v[0] * v[1]) & M32
+        elif op == "mulk_i32":
+            a0 = g(0)
+            if a0[1] != M32:
+                self._unknown_dest(wv, ops[0])
+                return
+            res = (a0[0] * sx(v[0], 16)) & M32
         elif op == "mul_hi_u32":
             res = ((v[0] * v[1]) >> 32) & M32
         elif op == "mul_hi_i32":

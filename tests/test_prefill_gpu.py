@@ -198,3 +198,21 @@ def test_a_run_of_any_length_alone_gives_its_bits_among_thousands(ctx, rows, wid
         np.testing.assert_array_equal(alone, whole[at[r] : at[r] + n])
         for got, want in zip(dec.read_cache(r, n), caches[r]):
             np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("rows, wide", [(1, False), (32, False), (1, True)])
+def test_a_run_by_any_rings_tiles_gives_its_bits_among_thousands(ctx, rows, wide):
+    """Lengths that take each of the rings (1, 2, 3, 4, 6 and 8 tiles a workgroup; the last workgroup's
+    tiles past the padded rows among them), alone and in one call of them all."""
+    from tgx.synth import StackSpec
+
+    lengths = (130, 193, 257, 321, 520, 700, 769, 1030) if wide else (256, 300, 500, 1100, 1167, 1536, 2600, 3073, 4100, 6200)
+    widths = dict(hidden=2048, inner=6144, head_dim=128) if wide else {}
+    spec = StackSpec(layers=2, dtype="bf16", **widths)
+    dec = make_decoder(ctx, spec, max(lengths), rows=rows, slots=max(rows, len(lengths)))
+    x = inputs(spec, sum(lengths))
+    at = np.cumsum([0, *lengths])
+    whole = dec.prefill_runs([(r, 0, n) for r, n in enumerate(lengths)], x)
+    for r, n in enumerate(lengths):
+        print(f"[prefill] {n} positions alone, {rows} rows, wide {wide}", flush=True)
+        np.testing.assert_array_equal(dec.prefill(0, x[at[r] : at[r] + n], slot=r), whole[at[r] : at[r] + n])

@@ -310,7 +310,7 @@ struct RingTile {
     static constexpr int LOADS = G * SW + XL;       // all its loads
     // The ring (the residual epilogue's rows take its place, HALF tiles at a time), then the rows'
     // scales.
-    static constexpr int HALF = TT < 4 ? TT : 4;
+    static constexpr int HALF = TT < 4 ? TT : TT % 4 ? 3 : 4;
     static constexpr int ROW_FLOATS = SPAN + 4;  // 16 rows' quads on different banks
     static constexpr size_t RING_BYTES = (size_t)R * G * TT * 1024, ROW_BYTES = (size_t)16 * HALF * ROW_FLOATS * 4;
     static constexpr size_t LDS = (RING_BYTES > ROW_BYTES ? RING_BYTES : ROW_BYTES) + 16 * TT * sizeof(float);
@@ -344,7 +344,7 @@ __device__ __forceinline__ void wait_loads(int n) {  // at most n (known once un
 }
 
 template <int EPI, int WR, int SW, int TT, int G, int R, int D>
-__global__ void __launch_bounds__(RING_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(RING_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(TT == 3 ? 1 : 2)))
 prefill_ring(PrefillArgs a, GemmArgs g, int NB, int MB) {
     using T = RingTile<SW, TT, G, R>;
     constexpr bool SCALED = !residual_epilogue(EPI);
@@ -352,6 +352,7 @@ prefill_ring(PrefillArgs a, GemmArgs g, int NB, int MB) {
     static_assert(EPI != EPI_SILU || SW == 2, "gate/up takes a gate strip and its up strip");
     static_assert(!residual_epilogue(EPI) || RING_WAVES * SW == SPAN_STRIPS, "a workgroup's columns are one span of a sum of squares");
     static_assert(ROWS <= RING_WAVES * WAVE, "a thread to a row");
+    static_assert(EPI != EPI_QKV || TT % 3, "the rows' places are read within the padded rows");
     extern __shared__ uint4 xs[];  // [R][G][TT tiles][64 lanes]
     float* scales = reinterpret_cast<float*>(reinterpret_cast<char*>(xs) + T::LDS) - ROWS;  // [ROWS]
     int nb, mb;
@@ -368,7 +369,7 @@ prefill_ring(PrefillArgs a, GemmArgs g, int NB, int MB) {
     float4 parts[MAX_SPANS / 4];
     const bool scaled = SCALED && g.row_sq && threadIdx.x < ROWS;
     if (scaled) {
-        const float* row = g.row_sq + (size_t)(m0 + threadIdx.x) * (g.K / SPAN);
+        const float* row = g.row_sq + (size_t)(TT % 3 ? m0 + threadIdx.x : min((uint32_t)m0 + threadIdx.x, (uint32_t)a.M_pad - 1u)) * (g.K / SPAN);
 #pragma unroll
         for (int i = 0; i < MAX_SPANS / 4; ++i) parts[i] = *reinterpret_cast<const float4*>(row + 4 * min(i, g.K / SPAN / 4 - 1));
     }
@@ -409,7 +410,9 @@ prefill_ring(PrefillArgs a, GemmArgs g, int NB, int MB) {
 #pragma unroll
         for (int j = 0; j < T::XL; ++j) {
             const int f = w * T::XL + j;
-            load_to_lds(g.x + ((size_t)(m0 / 16 + f % TT) * kblocks + st * G + f / TT) * 512 + lane * 8, &xs[(r * G * TT + f) * 64]);
+            // Three or six tiles may go past the padded rows: the last tile again, never stored.
+            const int tile = TT % 3 ? m0 / 16 + f % TT : __builtin_amdgcn_readfirstlane(min(m0 / 16 + f % TT, a.M_pad / 16 - 1));
+            load_to_lds(g.x + ((size_t)tile * kblocks + st * G + f / TT) * 512 + lane * 8, &xs[(r * G * TT + f) * 64]);
         }
     };
     // Each stage stays behind the stage before (the waits count loads in issue order).
@@ -582,28 +585,56 @@ void ring(const char* label, const PrefillArgs& a, const GemmArgs& g, hipStream_
 // The workgroups prefill_ring takes for M rows in tiles of 16 TT.
 int ring_groups(int M, int N, int TT) { return N / SPAN * ((M + 16 * TT - 1) / (16 * TT)); }
 
-// The ring with the fewest tiles a workgroup (the shortest chain a k-block) that still is one round of
-// a workgroup to each of the 256 CUs (down_proj at 384 rows: 17.8 us at one tile, 20.8 at two; 960
-// rows: 30.3, 20.9 and at four 23.2; 2048 rows: 37.9 at two, 25.2 at four, 37.8 at eight; gate/up, more
-// columns, from two tiles: 57 rows 7.7 at one, 8.0 at two). Past that eight tiles, whose operands take
-// less of the L2's rate (4096 rows: 63.5, 46.7, 42.0), until prefill_gemm's 256 x 128 tiles fill the
-// chip (down_proj 77.9 against 96.1 at 8192 rows, 158 against 139 at 16384; gate/up 32.8 against 33.7 at
-// 2048, 67.4 against 66.3 at 4096). q/k/v, whose epilogue leaves no registers for eight tiles, stays at
-// four with a k-block a stage (4096 rows 23.3 against 26.8 with two; 8192: 39.5, prefill_gemm 43.8;
-// 16384: 74.5, 70).
+// The tiles a workgroup, of the `n` counts in tts (fewest first), by which M rows take the fewest rounds of
+// a workgroup to each of the 256 CUs; the fewest tiles among equals, the shortest chain a k-block. us by
+// 1 / 2 / 3 / 4 / 6 / 8 tiles: down_proj at 500 rows 18.3 / 19.6 / 22.5 / 24.0 / 27.3 / 38.1, 960 rows 30.4 /
+// 20.6 / 22.2 / 23.4 / 30.1 / 38.4, 1167 rows - / 28.9 / 22.5 / 23.8 / 29.9 / 38.7, 2000 rows - / 38.0 / 39.2 /
+// 26.0 / 31.1 / 38.4, 2600 rows - / - / 41.6 / 37.8 / 32.9 / 39.8, 4000 rows - / - / 60.2 / 48.5 / 50.2 / 44.0, 5000
+// rows - / - / 78.0 / 62.2 / 53.7 / 59.7; gate/up at 300 rows 14.7 by two, 12.8 by four, 11.4 by six, 12.3 by
+// eight, 500 rows 18.9 / 14.0 / 15.6 / 12.5, 768 rows 23.8 / 20.2 / 17.4 / 18.0, 1167 rows 34.5 / 29.2 / 28.3 /
+// 27.0.
+int fewest_rounds(int M, int N, const int* tts, int n) {
+    int best = tts[0], rounds = (ring_groups(M, N, best) + 255) / 256;
+    for (int i = 1; i < n; ++i) {
+        const int r = (ring_groups(M, N, tts[i]) + 255) / 256;
+        if (r < rounds) {
+            best = tts[i];
+            rounds = r;
+        }
+    }
+    return best;
+}
+
+// The ring while its operands, read again by each workgroup, cost less than prefill_gemm's 256 x 128 tiles
+// leave idle (down_proj 77.9 against 96.1 us at 8192 rows, 158 against 139 at 16384; gate/up 32.3 against
+// 31.9 at 1600, 36.1 against 34.5 at 2000). q/k/v, whose epilogue leaves no registers for more, takes two
+// tiles or four with a k-block a stage (4096 rows 23.3 against 26.8 with two; 8192: 39.5, prefill_gemm
+// 43.8; 16384: 74.5, 70).
 template <int EPI, int WR, int D>
 hipError_t ring_by_rows(const char* label, const PrefillArgs& a, int strip_rows, const GemmArgs& g, hipStream_t stream, DispatchTimer* timer) {
-    constexpr bool QKV = EPI == EPI_QKV;
-    if (residual_epilogue(EPI) && ring_groups(a.M, g.N, 1) <= 256) {
-        if constexpr (residual_epilogue(EPI)) ring<EPI, WR, 1, 4, 4, D>(label, a, g, stream, timer);
-    } else if (ring_groups(a.M, g.N, 2) <= 256) {
-        ring<EPI, WR, 2, 2, 4, D>(label, a, g, stream, timer);
-    } else if (ring_groups(a.M, g.N, 4) <= (QKV ? 1280 : 256)) {
-        ring<EPI, WR, 4, QKV ? 1 : 2, QKV ? 8 : 4, D>(label, a, g, stream, timer);
-    } else if (!QKV && ring_groups(a.M, g.N, 8) <= 768) {
-        if constexpr (!QKV) ring<EPI, WR, 8, 1, 4, D>(label, a, g, stream, timer);
+    if constexpr (EPI == EPI_QKV) {
+        if (ring_groups(a.M, g.N, 2) <= 256)
+            ring<EPI, WR, 2, 2, 4, D>(label, a, g, stream, timer);
+        else if (ring_groups(a.M, g.N, 4) <= 1280)
+            ring<EPI, WR, 4, 1, 8, D>(label, a, g, stream, timer);
+        else
+            return launch_prefill_gemm(a, EPI, strip_rows, g, stream, timer);
     } else {
-        return launch_prefill_gemm(a, EPI, strip_rows, g, stream, timer);
+        if (ring_groups(a.M, g.N, 8) > 768) return launch_prefill_gemm(a, EPI, strip_rows, g, stream, timer);
+        constexpr int tts[] = {1, 2, 3, 4, 6, 8}, pairs[] = {2, 4, 6, 8};
+        int tt = residual_epilogue(EPI) ? fewest_rounds(a.M, g.N, tts, 6) : fewest_rounds(a.M, g.N, pairs, 4);
+        // Two full rounds of six tiles against eight's round and a half: o_proj 29.1 against 28.1 us at 6000
+        // rows (5000 rows, the second round less full: 23.9 against 26.8).
+        const int six = ring_groups(a.M, g.N, 6);
+        if (residual_epilogue(EPI) && tt == 6 && six > 256 && six * 8 > (six + 255) / 256 * 256 * 7) tt = 8;
+        if constexpr (residual_epilogue(EPI)) {
+            if (tt == 1) ring<EPI, WR, 1, 4, 4, D>(label, a, g, stream, timer);
+            if (tt == 3) ring<EPI, WR, 3, 4, 4, D>(label, a, g, stream, timer);
+        }
+        if (tt == 2) ring<EPI, WR, 2, 2, 4, D>(label, a, g, stream, timer);
+        if (tt == 4) ring<EPI, WR, 4, 2, 4, D>(label, a, g, stream, timer);
+        if (tt == 6) ring<EPI, WR, 6, 2, 4, D>(label, a, g, stream, timer);
+        if (tt == 8) ring<EPI, WR, 8, 1, 4, D>(label, a, g, stream, timer);
     }
     return hipGetLastError();
 }
