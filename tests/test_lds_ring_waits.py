@@ -214,6 +214,25 @@ def prefill_attention_case(symbol):
     check(runs, f"prefill_attention<{tile}, {waves}, {cg}, {d}> (group {group})")
 
 
+def test_prefill_attention_split_reads_no_chunk_before_it_lands():
+    symbols = instances(assembly("prefill_kernels.hip"), "prefill_attention_split")
+    assert len(symbols) >= 2, symbols  # head widths 64 and 128
+    for symbol in symbols:
+        part, waves, split, d = template_args(symbol)
+        k, L = assembly("prefill_kernels.hip")[symbol], layout("prefill_kernels.hip")
+        hidden, inner = (1024, 4096) if d == 64 else (2048, 6144)
+        whole = part * split
+        # A tile masked throughout, one well inside a run and one whose last part is ragged, each by its
+        # first part and its last for the last head.
+        tiles = [(0, 0, whole, 0), (whole, 333, whole, 0), (2 * whole, 700, whole - 1, 0)]
+        mem = rows_memory(3 * whole, 256, 16)
+        mem[TILES] = b"".join(struct.pack("<4I", *t) for t in tiles)
+        a = prefill_args(L, 3 * whole, 256, hidden, inner, 16, 2, d, 1024, 16, 16)
+        explicit = [a, struct.pack("<Q", Q), struct.pack("<Q", KV), struct.pack("<Q", ATT), struct.pack("<Q", TILES)]
+        wgs = [((split * t + s) * 2 + 1, 0, 0) for t in range(3) for s in (0, split - 1)]
+        check(replay(k, explicit, (6 * split, 1, 1), waves * 64, mem, wgs), f"prefill_attention_split<{part}, {waves}, {split}, {d}>")
+
+
 # ---- the local stack's ring GEMM ----
 
 LOCAL_EPI = {0: "qkv", 1: "partial", 2: "silu", 3: "add"}

@@ -698,11 +698,18 @@ constexpr int ATTN_STAGE = 2 * KV_TILE / 8;  // uint4: 16 fragments of 1 KiB
 constexpr int ATTN_STAGES = 4;
 constexpr int attention_chunk(int head_dim) { return head_dim == 64 ? BLOCK_TOKENS : BLOCK_TOKENS / 2; }
 
+// Whether a tile lies in the tensors: 1 to `most` positions, of a slot of the table, inside the cache's
+// capacity and the M_pad rows. One that does not is skipped by the whole workgroup before any barrier:
+// the host builds valid ones, and a caller's own tiles in device memory cannot be checked there.
+__device__ __forceinline__ bool tile_fits(const PrefillArgs& a, const PrefillTile& tile, uint32_t most) {
+    return !(tile.count == 0 || tile.count > most || tile.slot >= (uint32_t)a.nslots || tile.count > (uint32_t)a.capacity ||
+             tile.pos0 > (uint32_t)a.capacity - tile.count || tile.count > (uint32_t)a.M_pad || tile.row0 > (uint32_t)a.M_pad - tile.count);
+}
+
+// Tile `tile` of KV head kv.
 template <int TILE, int WAVES, int CG, int D>
-__global__ void __launch_bounds__(WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(2))) prefill_attention(PrefillArgs a, const uint16_t* __restrict__ q,
-                                                                 const uint16_t* __restrict__ kvpool,
-                                                                 uint16_t* __restrict__ attended,
-                                                                 const PrefillTile* __restrict__ tiles) {
+__device__ __forceinline__ void attend_tile(const PrefillArgs& a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kvpool,
+                                            uint16_t* __restrict__ attended, const PrefillTile& tile, int kv) {
     constexpr int THREADS = WAVES * WAVE;
     constexpr int TOK = TILE / WAVES;          // positions to a wave
     constexpr int per_col = TOK / CG;          // positions to a column group
@@ -723,10 +730,6 @@ __global__ void __launch_bounds__(WAVES * WAVE) __attribute__((amdgpu_waves_per_
     // slot's block ids.
     extern __shared__ uint4 attn_ring[];
     uint32_t* block_ids = reinterpret_cast<uint32_t*>(attn_ring + NS * ATTN_STAGE);
-    // Workgroup KV t + kv takes tile t for KV head kv: a tile's heads are dispatched together, in
-    // the tiles' order (the longest first), so that the last workgroups to start are short ones.
-    const int kv = (int)(blockIdx.x % (uint32_t)a.kv_heads);
-    const PrefillTile tile = tiles[blockIdx.x / (uint32_t)a.kv_heads];
     // A tile that leaves the tensors (1 to TILE positions, of a slot of the table, inside the
     // cache's capacity and the M_pad rows) is skipped by the whole workgroup before any barrier:
     // the host builds valid ones, and a caller's own tiles in device memory cannot be checked there.
@@ -899,6 +902,40 @@ __global__ void __launch_bounds__(WAVES * WAVE) __attribute__((amdgpu_waves_per_
     }
 }
 
+template <int TILE, int WAVES, int CG, int D>
+__global__ void __launch_bounds__(WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(2))) prefill_attention(PrefillArgs a, const uint16_t* __restrict__ q,
+                                                                 const uint16_t* __restrict__ kvpool,
+                                                                 uint16_t* __restrict__ attended,
+                                                                 const PrefillTile* __restrict__ tiles) {
+    // Workgroup KV t + kv takes tile t for KV head kv: a tile's heads are dispatched together, in
+    // the tiles' order (the longest first), so that the last workgroups to start are short ones.
+    const PrefillTile tile = tiles[blockIdx.x / (uint32_t)a.kv_heads];
+    if (!tile_fits(a, tile, TILE)) return;
+    attend_tile<TILE, WAVES, CG, D>(a, q, kvpool, attended, tile, (int)(blockIdx.x % (uint32_t)a.kv_heads));
+}
+
+// prefill_attention's tiles, of up to SPLIT TILE positions, cut: SPLIT workgroups to each, a wave one
+// column group where prefill_attention's takes two (at D 128 half as many waves). While the tiles leave a
+// CU to each workgroup a chunk costs a wave its own chain (keys from LDS, scores, softmax, values), not
+// the chip's rate: with half the columns 0.5 us in place of 0.75. Past that the chunks staged twice cost
+// more. us a launch at 300 / 1167 / 2048 positions of the backbone 6.9 / 15.5 / 24.3 -> 5.3 / 12.0 / 19.3
+// (two runs of 2048, 512 workgroups whole: 29.1 against 31.9), at 130 / 1000 of VoxCPM2's widths 6.9 / 20.1 ->
+// 5.8 / 18.7; a quarter to a workgroup of two waves 5.1 / 12.0 / 26.8.
+constexpr int ATTN_SPLIT = 2;
+constexpr uint32_t ATTN_SPLIT_MOST = 256;  // workgroups of whole tiles
+template <int TILE, int WAVES, int SPLIT, int D>
+__global__ void __launch_bounds__(WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(2))) prefill_attention_split(
+    PrefillArgs a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kvpool, uint16_t* __restrict__ attended,
+    const PrefillTile* __restrict__ tiles) {
+    const uint32_t t = blockIdx.x / (uint32_t)a.kv_heads, from = t % SPLIT * TILE;
+    PrefillTile tile = tiles[t / SPLIT];
+    if (!tile_fits(a, tile, SPLIT * TILE) || tile.count <= from) return;
+    tile.row0 += from;
+    tile.pos0 += from;
+    tile.count = min(tile.count - from, (uint32_t)TILE);
+    attend_tile<TILE, WAVES, 1, D>(a, q, kvpool, attended, tile, (int)(blockIdx.x % (uint32_t)a.kv_heads));
+}
+
 // Each projection's X rows to a workgroup. 128 for all: with two workgroups to a CU, one's
 // epilogue (10 bytes an output for o_proj and down_proj: the f32 residual in and out, the next
 // norm's bf16 operand) and prologue run beside the other's products, which at 8 x 2048 positions
@@ -934,6 +971,9 @@ hipError_t attention(const PrefillArgs& a, const uint16_t* q, const uint16_t* kv
     else if (group == 5) {
         if constexpr (D == 64) TGX_ATTENTION(ATTN_TILE_5, 4, 2);
         else TGX_ATTENTION(ATTN_TILE_5, 8, 1);
+    } else if (group > 5 && group <= 8 && grid.x <= ATTN_SPLIT_MOST) {
+        dispatch("prefill_attention", prefill_attention_split<ATTN_TILE_8 / ATTN_SPLIT, 4, ATTN_SPLIT, D>, dim3(ATTN_SPLIT * grid.x), dim3(4 * WAVE),
+                 lds, stream, timer, a, q, kv, attended, tiles);
     } else if (group <= 8) {
         if constexpr (D == 64) TGX_ATTENTION(ATTN_TILE_8, 4, 2);
         else TGX_ATTENTION(ATTN_TILE_8, 8, 1);
@@ -1061,7 +1101,9 @@ hipError_t prefill_prepare(size_t device_lds) {
                           (const void*)prefill_attention<ATTN_TILE, 8, 1, 128>, (const void*)prefill_attention<ATTN_TILE_8, 8, 1, 128>,
                           (const void*)prefill_attention<ATTN_TILE_16, 8, 2, 64>, (const void*)prefill_attention<ATTN_TILE_16_D128, 8, 1, 128>,
                           (const void*)prefill_attention<ATTN_TILE_3, 4, 2, 64>, (const void*)prefill_attention<ATTN_TILE_3, 8, 1, 128>,
-                          (const void*)prefill_attention<ATTN_TILE_5, 4, 2, 64>, (const void*)prefill_attention<ATTN_TILE_5, 8, 1, 128>})
+                          (const void*)prefill_attention<ATTN_TILE_5, 4, 2, 64>, (const void*)prefill_attention<ATTN_TILE_5, 8, 1, 128>,
+                          (const void*)prefill_attention_split<ATTN_TILE_8 / ATTN_SPLIT, 4, ATTN_SPLIT, 64>,
+                          (const void*)prefill_attention_split<ATTN_TILE_8 / ATTN_SPLIT, 4, ATTN_SPLIT, 128>})
         if ((e = allow(f, device_lds)) != hipSuccess) return e;
     return allow((const void*)prefill_gemm<EPI_SILU, QKV_ROWS, GATE_UP_TM>, device_lds);
 }

@@ -500,6 +500,7 @@ tgx_status build_attention_rows(const Bound* b, const uint32_t* c, Launch* L) {
     TGX_TRY(holds(b, 3, "tiles", (uint64_t)ntiles * sizeof(PrefillTile)));
     TGX_TRY(holds(b, 4, "attended", Mp * att * 2));
     a.table = (const uint32_t*)b[2].ptr;
+    L->also = dim3(ntiles * a.kv_heads);
     return capture_one("attention_rows", [&] {
         return launch_prefill_attention(a, (const uint16_t*)b[0].ptr, (const uint16_t*)b[1].ptr, (uint16_t*)b[4].ptr,
                                         (const PrefillTile*)b[3].ptr, (int)ntiles, nullptr, nullptr);
