@@ -1,5 +1,5 @@
 """The waits of the kernels that stage operands through LDS by direct global-to-LDS loads
-(prefill_gemm, prefill_attention, local_gemm_ring), checked on the compiler's own AMD assembly for
+(prefill_gemm, prefill_ring, prefill_attention, local_gemm_ring, local_gemm_parts), checked on the compiler's own AMD assembly for
 gfx950 by a replay of one workgroup's waves (tests/lds_replay.py): each kernel counts its loads in
 issue order (s_waitcnt vmcnt(N)) and reads LDS through inline asm the compiler does not order
 behind those loads, so the count is right only while the loads go out in the order the source

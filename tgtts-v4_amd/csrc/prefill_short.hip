@@ -343,6 +343,8 @@ __device__ __forceinline__ void wait_loads(int n) {  // at most n (known once un
     }
 }
 
+// Three tiles come four k-blocks a stage (a wave's share of fewer is not whole), whose operands are more
+// registers than two waves to a SIMD leave.
 template <int EPI, int WR, int SW, int TT, int G, int R, int D>
 __global__ void __launch_bounds__(RING_WAVES * WAVE) __attribute__((amdgpu_waves_per_eu(TT == 3 ? 1 : 2)))
 prefill_ring(PrefillArgs a, GemmArgs g, int NB, int MB) {
