@@ -1,0 +1,55 @@
+"""The library's host side on the CPU, over a stand-in for HIP's host calls (tests/hip_model.cpp): what
+it queues where, and what it waits for."""
+
+import pytest
+
+import hip_model
+
+
+@pytest.fixture(scope="module")
+def model(tmp_path_factory):
+    return hip_model.build(tmp_path_factory.mktemp("hip_model"))
+
+
+def test_memory_is_clear_before_anything_is_written_to_it(model):
+    """hipMemset may return before its fill has run, and the context's stream does not wait for the null
+    stream: a fill still on its way would take back what a write or a copy put there."""
+    hip_model.run(model, """
+        src, dst = rt.Memory(ctx, 4096), rt.Memory(ctx, 4096)
+        data = np.arange(1024, dtype=np.uint32)
+        src.write(data)
+        rt.copy_regions(ctx, dst, src, [(0, 2048, 1024)])
+        model.hip_model_settle()
+        assert np.array_equal(src.read(np.uint32, 1024), data)
+        want = np.zeros(1024, np.uint32)
+        want[512:768] = data[:256]
+        assert np.array_equal(dst.read(np.uint32, 1024), want)
+        assert model.hip_model_violations() == 0
+    """)
+
+
+def test_a_prefills_tensors_are_clear_before_its_rows_are_copied_in(model):
+    """The first prefill and each longer one allocate the tensors and clear them."""
+    hip_model.run(model, """
+        from tgx.synth import StackSpec
+        spec = StackSpec(layers=1, dtype="bf16")
+        shape = tgx.Shape(hidden=spec.hidden, inner=spec.inner, heads=spec.heads, kv_heads=spec.kv_heads,
+                          head_dim=spec.head_dim, layers=1, capacity=640)
+        dec = tgx.Decoder(ctx, shape, tgx.Batch(rows=1, slots=1))
+        for n in (3, 300, 600):
+            dec.prefill(0, np.ones((n, spec.hidden), np.float32))
+        assert model.hip_model_violations() == 0
+    """)
+
+
+def test_a_models_tensors_are_clear_when_it_is_created(model):
+    """No clear is left to run beside a new model's first copies and kernels."""
+    hip_model.run(model, """
+        from tgx.patch import Encoder, LmSide, PatchShape, Sampler
+        shape, patch = tgx.Shape(layers=1, capacity=64), PatchShape(64, 4, 2, 1)
+        kept = []  # destroying one waits for the device
+        for create in (lambda: tgx.Decoder(ctx, shape, tgx.Batch(rows=1, slots=1)), lambda: Sampler(ctx, shape, patch),
+                       lambda: Encoder(ctx, shape, patch), lambda: LmSide(ctx, shape, shape, tgx.Batch(rows=1, slots=1))):
+            kept.append(create())
+            assert model.hip_model_pending() == 0 and model.hip_model_violations() == 0, type(kept[-1])
+    """)

@@ -21,8 +21,7 @@ tgx_status encoder_alloc(Encoder* e, T** out, size_t count) {
     if (err != hipSuccess) return fail(TGX_E_HIP, "hipMalloc of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(err));
     e->allocations.push_back({p, bytes});
     e->device_bytes += bytes;
-    err = hipMemset(p, 0, bytes);
-    if (err != hipSuccess) return fail(TGX_E_HIP, std::string("hipMemset: ") + hipGetErrorString(err));
+    TGX_TRY(clear_memory(p, bytes));
     *out = (T*)p;
     return TGX_OK;
 }

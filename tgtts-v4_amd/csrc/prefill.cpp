@@ -51,14 +51,16 @@ tgx_status hold_rows(Decoder* d, int rows, int tiles) {
     TGX_TRY(prefill_alloc(d, &p.tok_pos, (size_t)rows));
     TGX_TRY(prefill_alloc(d, &p.tok_slot, (size_t)rows));
     TGX_TRY(prefill_alloc(d, &p.tiles, (size_t)tiles));
-    // Rows past a run's are read by the GEMMs: keep them zero.
-    TGX_HIP(hipMemset(p.x, 0, rows * h * 4));
-    TGX_HIP(hipMemset(p.h, 0, rows * h * 4));
-    TGX_HIP(hipMemset(p.mid, 0, rows * h * 4));
-    TGX_HIP(hipMemset(p.normed, 0, rows * h * 2));
-    TGX_HIP(hipMemset(p.row_sq, 0, rows * h / 128 * 4));
-    TGX_HIP(hipMemset(p.attended, 0, rows * att * 2));
-    TGX_HIP(hipMemset(p.mlp, 0, rows * (size_t)s.inner * 2));
+    // Rows past a run's are read by the GEMMs: keep them zero. On the context's stream, ahead of the
+    // prefill that asked for them.
+    hipStream_t st = d->ctx->stream;
+    TGX_HIP(launch_fill_zero(p.x, rows * h * 4, st));
+    TGX_HIP(launch_fill_zero(p.h, rows * h * 4, st));
+    TGX_HIP(launch_fill_zero(p.mid, rows * h * 4, st));
+    TGX_HIP(launch_fill_zero(p.normed, rows * h * 2, st));
+    TGX_HIP(launch_fill_zero(p.row_sq, rows * h / 128 * 4, st));
+    TGX_HIP(launch_fill_zero(p.attended, rows * att * 2, st));
+    TGX_HIP(launch_fill_zero(p.mlp, rows * (size_t)s.inner * 2, st));
     p.rows_held = rows;
     p.tiles_held = tiles;
     return TGX_OK;

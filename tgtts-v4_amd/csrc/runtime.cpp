@@ -95,6 +95,13 @@ void rope_tables(const Shape& s, std::vector<float>& cos, std::vector<float>& si
         }
 }
 
+tgx_status clear_memory(void* p, size_t bytes) {
+    hipError_t e = hipMemset(p, 0, bytes);
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
+    if (e != hipSuccess) return fail(TGX_E_HIP, std::string("clearing memory: ") + hipGetErrorString(e));
+    return TGX_OK;
+}
+
 tgx_status upload_graph(hipGraphExec_t exec, hipStream_t stream) {
     TGX_HIP(hipGraphUpload(exec, stream));
     TGX_HIP(hipStreamSynchronize(stream));
@@ -366,10 +373,7 @@ tgx_status alloc(Decoder* d, T** out, size_t count, bool zero = true) {
     if (e != hipSuccess) return fail(TGX_E_HIP, "hipMalloc of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
     d->allocations.push_back({p, bytes});
     d->device_bytes += bytes;
-    if (zero) {
-        e = hipMemset(p, 0, bytes);
-        if (e != hipSuccess) return fail(TGX_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
-    }
+    if (zero) TGX_TRY(clear_memory(p, bytes));
     *out = (T*)p;
     return TGX_OK;
 }

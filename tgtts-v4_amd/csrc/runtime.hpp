@@ -44,6 +44,10 @@ struct Context {
     uint64_t* clock_host = nullptr;   // pinned host word read_clock writes for tgx_context_calibrate
 };
 
+// Zeroes device memory, done when it returns: hipMemset may return before its fill has run, and the
+// contexts' streams do not wait for the null stream.
+tgx_status clear_memory(void* p, size_t bytes);
+
 // Waits for `ev`, recorded on the context's stream: polls it without pause for the context's
 // fence spin, then every 5 µs, for 60 s at most (Inner::wait_for, crates/vulkan/src/context.rs:
 // 116-133, and its FENCE_TIMEOUT_NS). TGX_E_HIP for an error the event reports, TGX_E_TIMEOUT

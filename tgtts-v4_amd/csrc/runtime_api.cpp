@@ -1233,10 +1233,10 @@ tgx_status tgx_alloc(tgx_context* ctx, uint64_t bytes, tgx_residence residence, 
     void* p = nullptr;
     if (residence == TGX_DEVICE) {
         TGX_HIP(hipMalloc(&p, bytes));
-        hipError_t e = hipMemset(p, 0, bytes);
-        if (e != hipSuccess) {
+        const tgx_status st = clear_memory(p, bytes);
+        if (st != TGX_OK) {
             hipFree(p);
-            return fail(TGX_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
+            return st;
         }
     } else {
         TGX_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));

@@ -71,8 +71,7 @@ tgx_status sampler_alloc(Sampler* s, T** out, size_t count) {
     if (e != hipSuccess) return fail(TGX_E_HIP, "hipMalloc of " + std::to_string(bytes) + " bytes: " + hipGetErrorString(e));
     s->allocations.push_back({p, bytes});
     s->device_bytes += bytes;
-    e = hipMemset(p, 0, bytes);
-    if (e != hipSuccess) return fail(TGX_E_HIP, std::string("hipMemset: ") + hipGetErrorString(e));
+    TGX_TRY(clear_memory(p, bytes));
     *out = (T*)p;
     return TGX_OK;
 }
