@@ -53,3 +53,28 @@ def test_a_models_tensors_are_clear_when_it_is_created(model):
             kept.append(create())
             assert model.hip_model_pending() == 0 and model.hip_model_violations() == 0, type(kept[-1])
     """)
+
+
+@pytest.mark.parametrize("inner", [1024, 4096])
+def test_a_gate_up_takes_the_grid_named_for_it_by_128s_of_tokens(model, inner):
+    """A caller that names local_gate_up's grid as it was first cut (past 64 tokens a workgroup to 64
+    columns and 128 tokens where the padded tokens come in 128s, else 64) is served whatever the kernel
+    takes; another grid is refused."""
+    hip_model.run(model, f"""
+        inner = {inner}
+        w = rt.Memory(ctx, 2 * inner * 1024 * 2)
+        for tokens in (17, 64, 65, 128, 192, 256, 320, 345, 384, 700):
+            pad = -(-tokens // 64) * 64 if tokens > 64 else -(-tokens // 16) * 16
+            x, sq, mlp = rt.Memory(ctx, pad * 1024 * 2), rt.Memory(ctx, pad * 16 * 4), rt.Memory(ctx, pad * inner * 2)
+            c = [tokens, 1, 1024, inner, 16, 2, rt.f32_bits(1e-5), 1]
+            step = 128 if pad % 128 == 0 else 64
+            first = (inner // 64, pad // step, 1) if tokens > 64 else (inner // 16, 1, 1)
+            for groups in ((0, 0, 0), first):
+                rt.dispatch(ctx, "local_gate_up", [x, w, sq, mlp], c, groups)
+            try:
+                rt.dispatch(ctx, "local_gate_up", [x, w, sq, mlp], c, (inner // 64, 40, 1))
+            except tgx.TgxError as e:
+                assert e.kind == "shape"
+            else:
+                assert False, tokens
+    """)

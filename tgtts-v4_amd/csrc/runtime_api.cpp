@@ -803,6 +803,7 @@ tgx_status build_local_gate_up(const Bound* b, const uint32_t* c, Launch* L) {
     g.N = 2 * a.inner;
     g.row_sq = (const float*)b[2].ptr;
     g.mlp = (uint16_t*)b[3].ptr;
+    if (a.M_pad > 64) L->also = dim3(a.inner / 64, a.M_pad % 128 == 0 ? a.M_pad / 128 : a.M_pad / 64);
     return capture_one("local_gate_up", [&] { return launch_local_gate_up(a, g, nullptr, nullptr); }, L);
 }
 
