@@ -78,3 +78,67 @@ def test_a_gate_up_takes_the_grid_named_for_it_by_128s_of_tokens(model, inner):
             else:
                 assert False, tokens
     """)
+
+
+@pytest.mark.parametrize("head_dim,capacity", [(64, 1152), (64, 2048), (128, 512), (128, 1024)])
+def test_no_step_records_a_program(model, head_dim, capacity):
+    """The programs of a decoder's rows are recorded when the rows are set, for steps with a row past
+    decode_far positions and without: recording waits for everything queued on the context. A capacity
+    that no such row fits has the one kind of program."""
+    hip_model.run(model, f"""
+        D, cap = {head_dim}, {capacity}
+        line = 1152 if D == 64 else 512
+        layers, h = 2, 1024 if D == 64 else 2048
+        dec = tgx.Decoder(ctx, tgx.Shape(hidden=h, inner=4 * h if h == 1024 else 6144, head_dim=D, layers=layers, capacity=cap),
+                          tgx.Batch(rows=2, slots=2))
+        recorded = model.hip_model_graphs()
+        assert recorded == (4 if cap > line else 2)
+        x = np.zeros((2, h), np.float32)
+        for position in [p for p in (0, line - 1, line, cap - 1, 0) if p < cap]:
+            dec.step_rows([tgx.Row(position, 0), None], x)
+            assert model.hip_model_last_nodes() == (6 if position >= line else 5) * layers + 1, position
+        for at in [p for p in (0, line - 2, cap - 3, 0) if p + 2 < cap]:
+            dec.set_rows([tgx.Row(at, 0), None], x)
+            dec.launch(3, advance=True)
+            dec.wait()
+            assert model.hip_model_last_nodes() == (6 if at + 2 >= line else 5) * layers + 1, at
+        assert model.hip_model_graphs() == recorded
+    """)
+
+
+@pytest.mark.parametrize("kv", [(2, 2), (2, 4)])
+def test_no_step_of_the_lm_side_records_a_program(model, kv):
+    """As above for both LMs at once, alone and in a patch step of fewer rows: at 20 rows an LM of 4 KV
+    heads (80 groups) has its line at 4096 positions, one of 2 at 1152."""
+    hip_model.run(model, f"""
+        from tgx.patch import Encoder, LmSide, PatchShape, PatchStep, Sampler
+        from tgx.synth import StackSpec, sampler_weights
+        kv, rows, C, F = {kv}, 20, 64, 4
+        lm = lambda kv: tgx.Shape(layers=1, kv_heads=kv, capacity=5000)
+        side = LmSide(ctx, lm(kv[0]), lm(kv[1]), tgx.Batch(rows=rows, slots=rows))
+        local, patch = tgx.Shape(layers=1, capacity=64), PatchShape(C, F, 2, rows)
+        sampler, encoder = Sampler(ctx, local, patch), Encoder(ctx, local, patch)
+        sampler.load_all(sampler_weights(StackSpec(layers=1, hidden=1024, inner=4096, dtype="bf16"), C))
+        step = PatchStep(encoder, side, sampler)
+        zeros = lambda *n: np.zeros(n, np.float32)
+        at = lambda n, position: [tgx.Row(position if r == 0 else 3, r) for r in range(n)]
+        for n in (rows, 3):
+            step.run_rows(at(n, 0), zeros(n, C, F), zeros(n, C, F), zeros(n, 2))
+            recorded = model.hip_model_graphs()
+            for position in (1151, 1152, 4096, 0):
+                step.run_rows(at(n, position), zeros(n, C, F), zeros(n, C, F), zeros(n, 2))
+                assert model.hip_model_graphs() == recorded, (n, position)
+        side.step_rows(at(rows, 0), zeros(rows, 1024))
+        recorded = model.hip_model_graphs()
+        for position in (1151, 1152, 4095, 4096, 0):
+            side.step_rows(at(rows, position), zeros(rows, 1024))
+            far = [position >= (4096 if rows * k > 64 else 1152) for k in kv]
+            assert model.hip_model_last_nodes() == 8 + sum(7 if f else 6 for f in far), position
+        for position in (1150, 4094):
+            side.set_rows(at(rows, position), zeros(rows, 1024))
+            side.launch(3, advance=True)
+            side.wait()
+            far = [position + 2 >= (4096 if rows * k > 64 else 1152) for k in kv]
+            assert model.hip_model_last_nodes() == 8 + sum(7 if f else 6 for f in far), position
+        assert model.hip_model_graphs() == recorded
+    """)

@@ -114,6 +114,22 @@ tgx_status side_program(LmSide* s) {
     return TGX_OK;
 }
 
+// Every program of s->rows rows recorded, a step's launch only picks one; the near one current. The two
+// LMs run the same rows, and differ in `far` only where their KV heads do.
+tgx_status record_programs(LmSide* s) {
+    Decoder *b = s->base, *r = s->residual;
+    const bool apart = b->shape.kv_heads != r->shape.kv_heads;
+    for (const bool base_far : {true, false})
+        for (const bool residual_far : {true, false}) {
+            if ((base_far && !decoder_can_go_far(b)) || (residual_far && !decoder_can_go_far(r)) || (base_far != residual_far && !apart))
+                continue;
+            b->far = base_far;
+            r->far = residual_far;
+            TGX_TRY(side_program(s));
+        }
+    return TGX_OK;
+}
+
 }  // namespace
 
 void destroy_programs(std::map<int, RowProgram>& programs) {
@@ -135,7 +151,7 @@ tgx_status lm_side_use_rows(LmSide* s, int rows) {
     if (st == TGX_OK) st = decoder_use_rows(s->residual, rows);
     if (st == TGX_OK) {
         s->rows = rows;
-        st = side_program(s);
+        st = record_programs(s);
     }
     if (st != TGX_OK) {
         // Back to the program it had (recorded already), with its message kept.
@@ -223,7 +239,7 @@ tgx_status lm_side_create(Context* ctx, const tgx_shape* base, const tgx_shape* 
     hipError_t e = hipEventCreate(&s->ev_start);
     if (e == hipSuccess) e = hipEventCreate(&s->ev_end);
     if (e != hipSuccess) return done(fail(TGX_E_HIP, std::string("hipEventCreate: ") + hipGetErrorString(e)));
-    if ((r = side_program(s)) != TGX_OK) return done(r);
+    if ((r = record_programs(s)) != TGX_OK) return done(r);
     *out = s;
     return TGX_OK;
 }

@@ -441,7 +441,19 @@ tgx_status use_program(Decoder* d) {
     return TGX_OK;
 }
 
+bool decoder_can_go_far(const Decoder* d) {
+    return (uint32_t)d->shape.capacity > decode_far(d->shape.kv_heads, d->shape.head_dim);
+}
+
 namespace {
+
+// Every program of the decoder's rows recorded, a step's launch only picks one; the near one current.
+tgx_status record_programs(Decoder* d) {
+    d->far = decoder_can_go_far(d);
+    TGX_TRY(use_program(d));
+    d->far = false;
+    return use_program(d);
+}
 
 tgx_status create_inner(Decoder* d, const tgx_batch* batch) {
     const Shape& s = d->shape;
@@ -542,7 +554,7 @@ tgx_status create_inner(Decoder* d, const tgx_batch* batch) {
     TGX_HIP(hipEventCreateWithFlags(&d->ev_done, hipEventDisableTiming));
     TGX_HIP(hipEventCreateWithFlags(&d->ev_staged, hipEventDisableTiming));
     TGX_HIP(hipDeviceSynchronize());
-    return use_program(d);
+    return record_programs(d);
 }
 
 }  // namespace
@@ -844,11 +856,11 @@ tgx_status decoder_use_rows(Decoder* d, int rows) {
     const int before = d->rows;
     const bool far = d->far;
     d->rows = rows;
-    d->far = false;  // until rows are placed
-    tgx_status st = use_program(d);
+    tgx_status st = record_programs(d);
     if (st != TGX_OK) {
-        d->rows = before;  // the program it had stays
+        d->rows = before;  // back to the program it had, recorded already
         d->far = far;
+        use_program(d);
         return st;
     }
     // Every row spare until placed again.

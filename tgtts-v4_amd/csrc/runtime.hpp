@@ -121,7 +121,7 @@ struct Decoder {
     bool table_dirty = true, rows_dirty = true;
     std::vector<int> slot_blocks;     // blocks each slot holds
     std::vector<uint32_t> free_list;  // blocks nobody holds
-    // the recorded step, a program per row count run (step_exec, advance_exec: the current one's)
+    // the recorded step, by row count and reach (step_exec, advance_exec: the current one's)
     struct Program {
         hipGraphExec_t step = nullptr, advance = nullptr;
         int dispatches = 0;
@@ -187,8 +187,11 @@ tgx_status sync_slots(Decoder* d);
 // placed row's blocks up to the last position the steps write, refusing (TGX_E_SHAPE) a row the
 // steps would take past the capacity, or a pool that runs out; and sets `far` for the steps.
 tgx_status hold_ahead(Decoder* d, int times, int advance);
-// The program of the decoder's rows and `far` as the current one, recorded if it has not been.
+// The program of the decoder's rows and `far` as the current one, recorded if it has not been: when
+// the decoder is created or its rows change, both of them, so that no step waits for a recording.
 tgx_status use_program(Decoder* d);
+// Whether the capacity holds a row past decode_far.
+bool decoder_can_go_far(const Decoder* d);
 // The host's copy of the placement moved on as an advancing step moves the rows on the device.
 void moved_on(Decoder* d, int times);
 tgx_status prefill_runs(Decoder* d, const tgx_run* runs, int nruns, const float* x, float* out);
