@@ -142,3 +142,25 @@ def test_no_step_of_the_lm_side_records_a_program(model, kv):
             assert model.hip_model_last_nodes() == 8 + sum(7 if f else 6 for f in far), position
         assert model.hip_model_graphs() == recorded
     """)
+
+
+@pytest.mark.parametrize("N", [16, 48, 1008, 1024, 1040])
+@pytest.mark.parametrize("rows", [1, 2, 17])
+def test_a_residuals_next_input_holds_its_last_half_block(model, N, rows):
+    """gemv_residual writes out_n in blocks of 32 columns, a row's 32 after another row's: where N ends
+    in half a block, the last row's half lies past rows x N. The bytes written up to it are what the
+    binding must hold, and no more."""
+    hip_model.run(model, f"""
+        N, rows, K = {N}, {rows}, 1024
+        last = max((n // 32 * rows + b) * 32 + n % 32 for n in range(N) for b in range(rows))
+        full = rt.Memory(ctx, 1 << 22)
+        c = [1024, 4096, 16, 2, rows, 64, rows, 1, rows, rt.f32_bits(1e-5), 1, 64, K, N, 4]
+        for short in (0, 2):
+            out_n = rt.Memory(ctx, 2 * (last + 1) - short)
+            try:
+                rt.dispatch(ctx, "gemv_residual", [full, full, full, full, full, out_n, full], c)
+            except tgx.TgxError as e:
+                assert short and e.kind == "shape" and "out_n" in str(e), str(e)
+            else:
+                assert not short
+    """)

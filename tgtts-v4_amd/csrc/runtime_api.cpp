@@ -269,7 +269,8 @@ tgx_status build_residual(const Bound* b, const uint32_t* c, Launch* L) {
     TGX_TRY(holds(b, 4, "out", R * N * 4));
     if (norm) {
         TGX_TRY(holds(b, 3, "next_gain", (uint64_t)N * 4));
-        TGX_TRY(holds(b, 5, "out_n", R * N * 2));
+        // In blocks of 32 columns, row after row: half a block at N's end lies 32 columns a row apart.
+        TGX_TRY(holds(b, 5, "out_n", (N % 32 ? ((uint64_t)(N / 32) * R + R - 1) * 32 + N % 32 : R * N) * 2));
         TGX_TRY(holds(b, 6, "out_sq", R * (N / Rs) * 4));
     }
     ResidualArgs r{};
