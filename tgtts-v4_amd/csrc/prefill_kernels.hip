@@ -706,7 +706,7 @@ __device__ __forceinline__ bool tile_fits(const PrefillArgs& a, const PrefillTil
              tile.pos0 > (uint32_t)a.capacity - tile.count || tile.count > (uint32_t)a.M_pad || tile.row0 > (uint32_t)a.M_pad - tile.count);
 }
 
-// Tile `tile` of KV head kv.
+// Tile `tile` of up to TILE positions, which the caller has checked (tile_fits), for KV head kv.
 template <int TILE, int WAVES, int CG, int D>
 __device__ __forceinline__ void attend_tile(const PrefillArgs& a, const uint16_t* __restrict__ q, const uint16_t* __restrict__ kvpool,
                                             uint16_t* __restrict__ attended, const PrefillTile& tile, int kv) {
@@ -730,12 +730,6 @@ __device__ __forceinline__ void attend_tile(const PrefillArgs& a, const uint16_t
     // slot's block ids.
     extern __shared__ uint4 attn_ring[];
     uint32_t* block_ids = reinterpret_cast<uint32_t*>(attn_ring + NS * ATTN_STAGE);
-    // A tile that leaves the tensors (1 to TILE positions, of a slot of the table, inside the
-    // cache's capacity and the M_pad rows) is skipped by the whole workgroup before any barrier:
-    // the host builds valid ones, and a caller's own tiles in device memory cannot be checked there.
-    if (tile.count == 0 || tile.count > (uint32_t)TILE || tile.slot >= (uint32_t)a.nslots || tile.count > (uint32_t)a.capacity ||
-        tile.pos0 > (uint32_t)a.capacity - tile.count || tile.count > (uint32_t)a.M_pad || tile.row0 > (uint32_t)a.M_pad - tile.count)
-        return;
     // The wave's index, uniform: the branches on it below are the whole wave's.
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int lane = threadIdx.x % WAVE;
