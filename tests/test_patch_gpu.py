@@ -172,12 +172,12 @@ def test_the_sampler_refuses_what_it_cannot_run(ctx):
 BASE_LAYERS, RESIDUAL_LAYERS, LATENT, LEVELS = 3, 2, 256, 9
 
 
-def _lm_side(ctx, rows, w):
+def _lm_side(ctx, rows, w, capacity=256):
     import tgx
     from tgx.patch import HeadsShape, LmSide
 
-    base = tgx.Shape(layers=BASE_LAYERS, capacity=256)
-    residual = tgx.Shape(layers=RESIDUAL_LAYERS, capacity=256, rope=False)
+    base = tgx.Shape(layers=BASE_LAYERS, capacity=capacity)
+    residual = tgx.Shape(layers=RESIDUAL_LAYERS, capacity=capacity, rope=False)
     side = LmSide(ctx, base, residual, tgx.Batch(rows=rows, slots=rows), HeadsShape(1024, 1024, LATENT, LEVELS))
     side.load_all(w)
     return side
@@ -533,3 +533,63 @@ def test_samplers_around_64_tokens_give_a_request_the_same_bits(ctx):
         s.close()
         most = got if most is None else most
         np.testing.assert_array_equal(got, most[:n])
+
+
+def test_a_row_far_into_its_cache_gives_its_bits_through_the_lm_side_and_the_patch_step(ctx):
+    """A row past 1152 positions takes the LMs' attention in chains, a program of the LM side's own; among
+    more than 64 (row, KV head) groups it takes one workgroup a group. Over the line and back, by single
+    steps, by launches that move it over the line and by patch steps: its bits among 40 rows."""
+    import tgx
+    from tgx.patch import PatchStep, patch_launch
+    from tgx.synth import encoder_weights, sampler_weights
+
+    rows, line, first = 40, 1152, 1150
+    espec, dspec = _encoder_spec(1), _dit_spec(1)
+    enc = _encoder(ctx, rows, espec, encoder_weights(espec, FEAT))
+    smp = _sampler(ctx, rows, dspec, sampler_weights(dspec, FEAT))
+    _, _, w = _lm_weights()
+    side = _lm_side(ctx, rows, w, capacity=1280)
+    rng = np.random.default_rng(31)
+    for which in (0, 1):
+        side.decoder(which).prefill(0, rng.standard_normal((first, 1024)).astype(np.float32) * 0.5)
+    _, cond, noise, sampling = _inputs(rows, seed=32)
+    embedding = enc.encode(cond)
+    near = side.dispatches()
+    alone = lambda position: [tgx.Row(position, 0)] + [None] * (rows - 1)
+    among = lambda position: [tgx.Row(position, 0)] + [tgx.Row(r % 5, r) for r in range(1, rows)]
+    far_layers = lambda position: BASE_LAYERS + RESIDUAL_LAYERS if position >= line else 0
+
+    want = {}
+    for position in range(first, first + 6):
+        mu, stop = side.step_rows(among(position), embedding)
+        want[position] = mu[0], stop[0]
+        assert side.dispatches() == near
+    for position in (*range(first, first + 6), first):
+        print(f"[lm_side] position {position} alone", flush=True)
+        mu, stop = side.step_rows(alone(position), embedding)
+        assert side.dispatches() == near + far_layers(position)
+        assert np.array_equal(mu[0], want[position][0]) and np.array_equal(stop[0], want[position][1]), position
+    side.set_rows(alone(first), embedding)
+    side.launch(4, advance=True)
+    side.wait()
+    assert side.dispatches() == near + far_layers(line)
+    assert np.array_equal(side.read("mu")[0], want[first + 3][0])
+    side.set_rows(alone(first), embedding)
+    patch_launch(side, smp, 3)
+    side.wait()
+    assert np.array_equal(side.read("mu")[0], want[first + 2][0])
+
+    step = PatchStep(enc, side, smp)
+    patches = {p: step.run_rows(among(p), cond, noise, sampling) for p in (first, line - 1, line, line + 1)}
+    for position in (line - 1, line, line + 1, first):
+        print(f"[patch] position {position} alone", flush=True)
+        for at in ([tgx.Row(position, 0)], alone(position)):  # the program of one row, and of them all
+            n = len(at)
+            patch, stop = step.run_rows(at, cond[:n], noise[:n], sampling[:n])
+            assert np.array_equal(patch[0], patches[position][0][0]) and np.array_equal(stop[0], patches[position][1][0]), (position, n)
+    step.launch(3, advance=True)  # from `first`, of all the rows' program
+    step.wait()
+    assert np.array_equal(side.read("mu")[0], want[first + 2][0])
+    step.close()
+    for o in (enc, smp, side):
+        o.close()
