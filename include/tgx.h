@@ -69,7 +69,9 @@ tgx_status tgx_context_report(const tgx_context* ctx, tgx_device_report* out);
 /* Context::set_fence_spin (crates/vulkan/src/context.rs:467-474, its wait Inner::wait_for,
  * :116-133): every wait for the context's work (tgx_decoder_wait, tgx_program_wait and the
  * sampler's, LM side's, encoder's and patch step's) polls for up to `ns` nanoseconds before it
- * sleeps between polls, 5 µs apart, 60 s at most in all; 0, the default, sleeps at once. */
+ * sleeps between polls, 5 µs apart, 60 s at most in all; 0, the default, sleeps at once. While it
+ * sleeps the calling thread's timer slack is at most 1 µs (it gets its own back with the result),
+ * and the thread takes about a third of a host core; while it polls, a whole one. */
 tgx_status tgx_context_set_fence_spin(tgx_context* ctx, uint64_t ns);
 /* Calibration (context.rs:73-88): the GPU's clock read `ticks` while the host's CLOCK_MONOTONIC
  * read `monotonic_ns`, give or take `deviation_ns`; `period_ns` nanoseconds a tick. */

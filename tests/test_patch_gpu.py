@@ -98,8 +98,8 @@ def test_a_row_samples_the_same_patch_beside_others_as_alone(ctx):
     w = sampler_weights(spec, FEAT)
     mu, cond, noise, sampling = _inputs(16, seed=9)
     one = _sampler(ctx, 1, spec, w)
-    # 1 row (22 tokens) takes the direct GEMMs; 5 rows (110 tokens, 128 padded) and 16 (352, 384)
-    # the ring GEMMs with 8 token tiles to a gate/up workgroup, 6 rows (132, 192) with 4.
+    # 1 row (22 tokens) takes the direct GEMMs; 5 rows (110 tokens, 128 padded) and 6 (132, 192) the
+    # ring GEMMs with 4 token tiles to a gate/up workgroup, 16 rows (352, 384) with 8.
     for rows, picks in ((5, (0, 3)), (6, (5,)), (16, (0, 9, 15))):
         many = _sampler(ctx, rows, spec, w)
         got = many.sample(mu[:rows], cond[:rows], noise[:rows], sampling[:rows])
@@ -114,7 +114,7 @@ def test_a_row_samples_the_same_patch_beside_others_as_alone(ctx):
 
 def test_repeated_samples_are_the_same_bits(ctx):
     """The same inputs sampled again and again give the same bits: at 5 rows (128 tokens, the ring
-    GEMM with 4 and 8 token tiles) and 16 rows (384), every workgroup's loads, waits and barriers
+    GEMM with 4 token tiles) and 16 rows (384, with 4 and 8), every workgroup's loads, waits and barriers
     read what they wait for (a race would show as a sample that differs from the first)."""
     from tgx.synth import sampler_weights
 
@@ -473,7 +473,7 @@ def test_fresh_patch_steps_beside_used_ones_give_a_warm_steps_bits_on_their_firs
 @pytest.mark.parametrize("feat,frames,rows", [(64, 4, (1, 3, 4, 12, 13)), (16, 1, (1, 8, 32, 33)), (48, 3, (2, 16, 17)), (32, 2, (1, 21, 22))])
 def test_an_encoder_of_any_rows_matches_the_oracle_and_gives_the_same_bits(ctx, feat, frames, rows):
     """The local stack on both sides of its line at 64 tokens (o_proj and down_proj by local_gemm_sum
-    up to it, by the ring past it), at part-filled tiles, and the embedding at every count of frames
+    up to it, by local_gemm_parts past it), at part-filled tiles, and the embedding at every count of frames
     and of channels: each row against the oracle, and the same bits whatever its encoder's rows."""
     import patch_oracle as po
     import tgx
@@ -520,7 +520,8 @@ def test_a_sampler_of_many_rows_gives_a_request_its_bits_alone(ctx, rows):
 
 
 def test_samplers_around_64_tokens_give_a_request_the_same_bits(ctx):
-    """Two requests' 44 tokens go through the kernels for at most 64, three's 66 through the ring's."""
+    """Two requests' 44 tokens go through the kernels for at most 64, three's 66 through the ring's and
+    (o_proj and down_proj) local_gemm_parts."""
     from tgx.synth import sampler_weights
 
     spec = _dit_spec(layers=2)

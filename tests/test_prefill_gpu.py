@@ -176,7 +176,7 @@ def test_nan_left_in_a_reused_block_past_the_run_never_reaches_its_outputs(ctx):
 @pytest.mark.parametrize("rows,wide", [(1, False), (32, False), (8, True)])
 def test_a_run_of_any_length_alone_gives_its_bits_among_thousands(ctx, rows, wide):
     """A short run's projections take kernels of their own (prefill_short.hip: strips by tiles a
-    wave, rings of 1, 2, 4 and 8 tiles); among thousands of positions the same rows go
+    wave, rings of 1 to 8 tiles); among thousands of positions the same rows go
     through larger tiles. Lengths on both sides of every line between those kernels, at the decode
     strip heights 4 and 16 (1 and 32 rows) and at VoxCPM2's widths: outputs and cache exactly
     alike."""

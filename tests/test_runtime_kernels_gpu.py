@@ -6,7 +6,7 @@ as the library's own run of the same work:
   output rows and the cache both layers wrote;
 - one DiT evaluation (a sample of 2 timesteps: one Euler step past CFG-Zero*'s zero init) against
   tgx_sampler_sample, at 1 row (22 tokens: the GEMMs' direct path, local_partial and
-  local_add_norm) and 3 rows (66 tokens: the ring, local_gemm_add_norm).
+  local_add_norm) and 3 rows (66 tokens: the ring, and local_gemm_parts by local_gemm_add_norm).
 
 Workload: MiniCPM-4-shaped stacks at hidden 1024 (16/2 heads of 64, FFN 4096); the prefill's
 cache of 256 positions in 2 slots; the sampler's patches of 4 frames x 64 channels."""

@@ -94,7 +94,8 @@ int decode_max_capacity(int head_dim);
 // step of 24 layers one way and the other: one row at 1000 positions 666 and 672, at 1200 710 and
 // 680, at 3000 898 and 727; 16 rows at 1200 757 and 744; four layers at head_dim 128, 8 rows at 500
 // 262 and 254. Past 64 groups the one workgroup each already fills the chip: 64 rows at 2100 999 and
-// 998, at 4000 1292 and 1301, up to 8000 1718 and 1451.
+// 998, at 4000 1292 and 1301, up to 8000 1718 and 1451. Every row at the one position, that is: among
+// more than 64 groups a lone row between the lines stays with the one workgroup, its place not timed.
 constexpr uint32_t decode_far(int groups, int head_dim) { return groups > 64 ? 4096 : head_dim == 64 ? 1152 : 512; }
 constexpr uint32_t DECODE_FAR_LEAST = 512;
 size_t decode_chain_floats(const DecodeArgs& a);

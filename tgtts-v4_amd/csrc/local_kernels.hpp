@@ -93,8 +93,9 @@ struct EulerArgs {
 };
 
 // What a local stack's projection writes beside its products (local_gemm_direct, local_gemm_ring):
-// q/k/v with RoPE, the parts of a sum (o_proj and down_proj up to 64 tokens), SiLU(gate) up, or
-// the parts added with the residual and the next norm's input (o_proj and down_proj past 64).
+// q/k/v with RoPE, the parts of a sum (by name, up to 64 tokens), SiLU(gate) up, or the parts added
+// with the residual and the next norm's input (o_proj and down_proj; local_gemm_sum's and
+// local_gemm_parts' only epilogue).
 enum LocalEpilogue { LEPI_QKV = 0, LEPI_PARTIAL = 1, LEPI_SILU = 2, LEPI_ADD = 3 };
 
 // A local projection's operands and its epilogue's tensors.
@@ -108,8 +109,8 @@ struct LocalGemm {
     // LEPI_QKV, LEPI_SILU: X is an RMSNorm's input times its gain; row m's sums of squares
     // [M_pad][K / LOCAL_SQ_COLS] give the row's scale, applied to its sums.
     const float* row_sq;
-    // LEPI_ADD (local_gemm_ring, local_gemm_sum): sum = residual + the parts' sums, and with next_gain, the next
-    // norm's input: normed = sum next_gain in bf16 and sum's sums of squares into sum_sq.
+    // LEPI_ADD: sum = residual + the parts' sums, and with next_gain, the next norm's input: normed =
+    // sum next_gain in bf16 and sum's sums of squares into sum_sq.
     const float* residual;
     float* sum;
     const float* next_gain;
@@ -120,9 +121,10 @@ struct LocalGemm {
 };
 
 // The local stack's kernels one at a time, as launch_local_stack launches them: q/k/v with RoPE
-// (its N the q/k/v rows), the attention within each sequence, o_proj's or down_proj's parts
-// (up to 64 tokens) and their sum with the residual and the next norm's input (or the final norm
-// into `out`), the same fused (2 or 4 parts; g.fine up to 64 tokens), and gate/up with SiLU.
+// (its N the q/k/v rows), the attention within each sequence, o_proj and down_proj with the residual
+// and the next norm's input (launch_local_add: 2 or 4 parts; g.fine up to 64 tokens), the final norm
+// into `out` (launch_local_add_norm), and gate/up with SiLU; and by name only, the parts (up to 64
+// tokens) and their sum in dispatches of their own.
 hipError_t launch_local_qkv(const LocalArgs& a, const LocalGemm& g, hipStream_t stream, DispatchTimer* timer);
 hipError_t launch_local_attention(const LocalArgs& a, const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* attended,
                                   hipStream_t stream, DispatchTimer* timer);
@@ -133,7 +135,7 @@ hipError_t launch_local_add_norm(const LocalArgs& a, bool final, const float* pa
 hipError_t launch_local_add(const LocalArgs& a, const LocalGemm& g, int parts, hipStream_t stream, DispatchTimer* timer);
 hipError_t launch_local_gate_up(const LocalArgs& a, const LocalGemm& g, hipStream_t stream, DispatchTimer* timer);
 
-// Lets the ring GEMM take its rings of token tiles (up to 66 KiB) in LDS; once per process.
+// Lets the GEMMs take their rings of token tiles (up to 97 KiB) in LDS; once per process.
 hipError_t local_prepare();
 // The stacks the kernels take: hidden 1024, query heads a multiple of 4, and o_proj's and
 // down_proj's columns in 2 or 4 parts of 16 or 32 k-blocks of 32 columns each.
