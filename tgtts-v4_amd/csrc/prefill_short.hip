@@ -299,10 +299,10 @@ __global__ void __launch_bounds__((direct_waves<EPI, TT>() * WAVE)) prefill_dire
 // span of a sum of squares. What bounds it: a k-block takes a CU 290 cycles at two tiles (10 KiB of
 // operands; 16 or 240 workgroups, R 4 or 8 alike) and 640 at eight (16 KiB), and past a workgroup a
 // CU the operands come from L2 at 18.5 TB/s in all (whole launches, start and epilogue in them, average
-// 9 to 12 by the counters, gate/up and down_proj at 300 and 1167 rows). us a launch at the backbone against prefill_gemm:
-// 57 rows o_proj 25.1 -> 7.0, gate/up 18.9 -> 7.9; 960 rows q/k/v 27.9 -> 12.5, o_proj 27.9 -> 8.8,
-// gate/up 20.4 -> 18.7, down_proj 77.1 -> 20.9; 2048 rows 28.3 -> 16.6, 29.4 -> 12.0, 33.7 -> 32.4,
-// 78.2 -> 25.2; 8192 rows down_proj 96.1 -> 77.9.
+// 9 to 12 by the counters, gate/up and down_proj at 300 and 1167 rows). us a launch at the backbone
+// against prefill_gemm: 57 rows o_proj 25.1 -> 7.0, gate/up 18.9 -> 7.9; 960 rows q/k/v 27.9 -> 12.5,
+// o_proj 27.9 -> 8.8, gate/up 20.4 -> 18.7, down_proj 77.1 -> 20.9; 2048 rows 28.3 -> 16.6, 29.4 -> 12.0,
+// 33.7 -> 32.4, 78.2 -> 25.2; 8192 rows down_proj 96.1 -> 77.9.
 constexpr int RING_WAVES = 4;
 
 template <int SW, int TT, int G, int R>
